@@ -460,7 +460,7 @@ def main():
     nvec = (ns + 1) // 2
     if args.kernels_only:
         k = ctx.bench_hpsi(sep.SEP_PREC_FP32, nvec, ms, 5)
-        # the fused kernel's previous (xor-swizzled LDS) form, for comparison
+        # the xy-plane form (swizzled LDS placement), for comparison
         ctx.set_hpsi_family(sep.SEP_PREC_FP32, sep.SEP_HPSI_PLANE_SWIZZLED)
         k_swz = ctx.bench_hpsi(sep.SEP_PREC_FP32, nvec, ms, 5)
         ctx.set_hpsi_family(sep.SEP_PREC_FP32, sep.SEP_HPSI_PLANE)
@@ -587,12 +587,11 @@ def main():
     # i.e. N (7c + r) per complex vector and H application.  Where the filter
     # loop fuses pass C with the next step's pass A (the live timing then
     # reports pass A as 0), that kernel reads T, psi_{j-1}, V and writes
-    # psi_j and the next T: (4c + r) N nvec, and a step moves N (6c + r).
-    def roof(live, c, r, lines=False):
-        # lines: the row + strided-line family, whose fused step's spectral
-        # part is y lines, z pencils and y lines (3 x 2c per point)
+    # psi_j and the next T: (4c + r) N nvec, and a step moves N (6c + r).  The
+    # two-kernel form's tile and row kernels move the same as B and CA.
+    def roof(live, c, r):
         if live[0] <= 0.0:
-            per = {"B": (6 if lines else 2) * c * N * nvec, "CA": (4 * c + r) * N * nvec}
+            per = {"B": 2 * c * N * nvec, "CA": (4 * c + r) * N * nvec}
             tms = {"B": live[1], "CA": live[2]}
         else:
             per = {"A": 2 * c * N * nvec, "B": 2 * c * N * nvec, "C": (3 * c + r) * N * nvec}
@@ -616,12 +615,9 @@ def main():
 
     r32 = roof(live32, 8, 4)
     dom = max((q for q in r32 if not q.startswith("step")), key=lambda q: r32[q]["ms"])
-    fused = {sep.SEP_HPSI_PLANE: "k_plane_bwd_fwd_s<1024>",
-             sep.SEP_HPSI_PLANE_SWIZZLED: "k_plane_bwd_fwd_w<float,128>",
-             sep.SEP_HPSI_PLANE_CHUNKED: "k_plane_bwd_fwd_h<float,128>"}.get(
-                 ctx.hpsi_family(sep.SEP_PREC_FP32), "k_rows_bwd_fwd<float,128>")
-    kname = {"A": "k_plane_fwd_w<float,128>", "B": "k_pencil<float,128>",
-             "C": "k_plane_bwd_w<float,128>", "CA": fused}[dom]
+    kname = {"A": "k_xrows_fwd<float,128,16>", "B": "k_tile<float,8,4,128>",
+             "C": "k_xrows_bwd<float,128,16,false,false>",
+             "CA": "k_xrows_bwd<float,128,16,true,false>"}[dom]
     traffic = measured_traffic(kname, n, nvec)
     probe = round(ctx.bench_copy(4 << 30, 5), 1)  # plain 16 B/lane copy, best of 4 grids
     roofline = {"bound": "hbm", "kernel": kname, "achieved": r32[dom]["GBs"],
@@ -731,10 +727,7 @@ def main():
         "complex_hpsi_per_s": round(v32 / 2, 1),
         "roofline": roofline,
         "roofline_passes_fp32": r32,
-        # complex128 plane kernels exist up to 96 points per line; 128 runs the
-        # row + line family
-        "roofline_passes_fp64": (roof(live64, 16, 8, lines=n not in (16, 24, 32, 36, 48, 64, 96))
-                                 if live64 is not None else None),
+        "roofline_passes_fp64": roof(live64, 16, 8) if live64 is not None else None,
         "accum_ms_per_block": {"fp32": round(live32[3], 4),
                                "fp64": round(live64[3], 4) if live64 is not None else None},
         "fp32_pipeline_check": check,

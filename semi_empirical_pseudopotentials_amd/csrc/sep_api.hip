@@ -300,15 +300,6 @@ int sep_open(const sep_grid_desc *g, sep_ctx **out) {
       return SEP_ERR_HIP;
     }
   }
-  if (const long twb = plane_sep_tw_bytes(c->gd.nx, SEP_PREC_FP32)) {
-    std::vector<char> tws(twb);
-    plane_sep_tw_host(tws.data());
-    if (hipMalloc(&c->gd.twsep32, twb) != hipSuccess ||
-        hipMemcpy(c->gd.twsep32, tws.data(), twb, hipMemcpyHostToDevice) != hipSuccess) {
-      sep_close(c);
-      return SEP_ERR_HIP;
-    }
-  }
   c->gd.kxx = tabs_d[0];
   c->gd.kyy = tabs_d[1];
   c->gd.kzz = tabs_d[2];
@@ -326,7 +317,6 @@ int sep_close(sep_ctx *c) {
     if (c->gd.tw64[a]) hipFree(c->gd.tw64[a]);
     if (c->gd.tw32[a]) hipFree(c->gd.tw32[a]);
   }
-  if (c->gd.twsep32) hipFree(c->gd.twsep32);
   for (void *p : {(void *)c->gd.kxx, (void *)c->gd.kyy, (void *)c->gd.kzz, (void *)c->pot64,
                   (void *)c->pot32, (void *)c->states, (void *)c->states2, c->tb, (void *)c->scr,
                   (void *)c->gwork, c->ring})
@@ -842,10 +832,9 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   f.j = 1;
   // pass A of psi_0; every later pass A runs fused with the previous pass C
   f.so = so;
-  // spinors: V_so joins psi_j in the fused kernel's epilogue where the FP64
-  // whole-plane family runs; elsewhere the steps run unfused
-  const bool so_fused = sizeof(R) == 8 && c->so.pmap && c->so.natom > 0 &&
-                        hpsi_plane_family(c->gd, SEP_PREC_FP64);
+  // spinors: V_so joins psi_j in the row kernel's epilogue where the FP64
+  // split form runs; elsewhere the steps run unfused
+  const bool so_fused = sizeof(R) == 8 && c->so.pmap && c->so.natom > 0 && hpsi_so_fused(c->gd);
   f.fused = (!so || so_fused) && nc > 1 && !c->gd.no_fuse && hpsi_fused_supported<R>(c->gd);
   if (f.fused) {
     VecView<R> v0{f.ring, f.ring + ss, nullptr, 2 * ss};
@@ -2165,7 +2154,8 @@ extern "C" int sep_autotune(sep_ctx *c, int precision, long nvec, double *ms_pla
     // the filter loop's split step (spectral passes + fused kernel)
     tp = k[5] > 0.0 && !c->gd.no_fuse ? k[5] : k[4];
   }
-  c->gd.force_lines[precision] = true;
+  // a grid outside the plane family keeps its one form (see sep_set_hpsi_family)
+  c->gd.force_lines[precision] = tp > 0.0 || had;
   const int rc = precision == SEP_PREC_FP64 ? bench_impl<double>(c, nvec, 1, 5, k)
                                             : bench_impl<float>(c, nvec, 1, 5, k);
   if (rc != SEP_OK) {
@@ -2173,7 +2163,7 @@ extern "C" int sep_autotune(sep_ctx *c, int precision, long nvec, double *ms_pla
     return rc;
   }
   tl = k[5] > 0.0 && !c->gd.no_fuse ? k[5] : k[4];
-  c->gd.force_lines[precision] = !(tp > 0.0 && tp <= tl);
+  if (tp > 0.0) c->gd.force_lines[precision] = !(tp <= tl);
   if (ms_plane) *ms_plane = tp;
   if (ms_lines) *ms_lines = tl;
   return SEP_OK;
@@ -2288,7 +2278,11 @@ extern "C" int sep_set_hpsi_family(sep_ctx *c, int precision, int family) {
       return SEP_OK;
     }
     case SEP_HPSI_LINES:
-      c->gd.force_lines[precision] = true;
+      // where the grid has no plane family, its default form (the two-kernel
+      // split) stands for this one: the five-pass kernels are slower on every
+      // such grid, and the autotuner would otherwise have to fall back on them
+      c->gd.force_lines[precision] = plane_supported(c->gd.nx, c->gd.ny, precision) ||
+                                     getenv("SEP_FORCE_LINE_KERNELS") != nullptr;
       c->gd.fused_form[precision] = SEP_FUSED_PLANE;
       return SEP_OK;
   }

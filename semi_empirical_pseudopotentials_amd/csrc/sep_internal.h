@@ -16,20 +16,19 @@ struct GridDev {
   long N;
   void *tw64[3];  // exp(-2 pi i m/n) per axis, complex128
   void *tw32[3];  // same, complex64
-  void *twsep32;  // per-thread-index twiddles of the separable fused kernel (null if none)
   double *kxx, *kyy, *kzz;  // filter/init.c:125-135 axis tables (1/N folded in)
   double ekin;              // Ekinmax / N (filter/init.c:137)
   // pden > 0 turns pass B into the kinetic preconditioner: the spectrum is
   // multiplied by pnum / (kin + pden) instead of kin (kin with 1/N folded in)
   double pnum, pden;
   // per precision (SEP_PREC_FP64 = 0, SEP_PREC_FP32 = 1): use the row/line
-  // kernels even where a plane kernel exists (sep_autotune, or the test hook
+  // kernels (sep_set_hpsi_family, sep_autotune, or the test hook
   // SEP_FORCE_LINE_KERNELS)
   bool force_lines[2];
-  // the filter loop runs pass C and the next pass A as separate kernels
-  // (test hook SEP_SEPARATE_PASSES) instead of the fused plane kernel
+  // the filter loop runs each step's last and the next step's first kernel
+  // separately (test hook SEP_SEPARATE_PASSES) instead of fused
   bool no_fuse;
-  // per precision: the form of the fused plane kernel (SEP_FUSED_*)
+  // per precision: the form beside rows + lines (SEP_FUSED_*)
   int fused_form[2];
 };
 
@@ -82,34 +81,28 @@ int axpby_dev(double a, const double *x, double b, double *y, long n, hipStream_
 
 bool hop_supported(int n);
 bool plane_supported(int nx, int ny, int prec);
-// Forms of the fused plane kernel (pass C + next pass A):
-//   SEP_FUSED_PLANE     the fastest whole-plane form the grid has (the
-//                       separable placement at complex64 128^2, else the
-//                       swizzled one)
-//   SEP_FUSED_CHUNKED   half a plane of LDS, two workgroups per CU
-//   SEP_FUSED_SWIZZLED  the whole-plane kernel on the swizzled placement
+// Forms of H.psi beside rows + lines:
+//   SEP_FUSED_PLANE     the default: the two-kernel form (sep_split.h)
+//   SEP_FUSED_CHUNKED   complex64 128^2 xy planes, the fused kernel through
+//                       half a plane of LDS, two workgroups per CU
+//   SEP_FUSED_SWIZZLED  the same through a whole plane of LDS
 enum { SEP_FUSED_PLANE = 0, SEP_FUSED_CHUNKED = 1, SEP_FUSED_SWIZZLED = 2 };
 bool plane_fused_form_supported(int n, int prec, int form);
-// Bytes of the separable fused kernel's twiddle table for planes of n (0 if
-// that kernel does not exist for n / prec), and its host construction.
-long plane_sep_tw_bytes(int n, int prec);
-void plane_sep_tw_host(void *tab);
-
 template <typename R>
 int hpsi_prepare(const GridDev &gd);
 template <typename R>
 int hpsi_apply(const GridDev &gd, const VecView<R> &in, const VecView<R> &out, cx<R> *tb,
                const R *pot, int nvec, double alpha, double beta, double *part, long *nblk,
                hipStream_t st, hipEvent_t *ev = nullptr);
-// Split Newton step (sep_hpsi.hip): pass A alone, then per step pass B and
-// pass C fused with the next step's pass A (fwd_next); tb carries the
-// spectrum of the newest vector between calls.
+// Split Newton step (sep_hpsi.hip): the forward pass alone, then per step the
+// spectral passes and the last pass fused with the next step's forward one
+// (fwd_next); tb carries the spectrum of the newest vector between calls.
 template <typename R>
 bool hpsi_fused_supported(const GridDev &gd);
 template <typename R>
 int hpsi_fwd(const GridDev &gd, const VecView<R> &in, cx<R> *tb, int nvec, hipStream_t st);
-// spinor filter step: psi_j += alpha (V_so psi_{j-1}) inside the fused
-// kernel's epilogue (FP64 whole-plane family, not the last step): map[g] the
+// spinor filter step: psi_j += alpha (V_so psi_{j-1}) inside the row
+// kernel's epilogue (FP64 split form, not the last step): map[g] the
 // row of g (4 doubles per spinor) in g, or -1
 struct SoEpi {
   const int *map;
@@ -121,8 +114,8 @@ template <typename R>
 int hpsi_step(const GridDev &gd, const VecView<R> &in, const VecView<R> &out, cx<R> *tb,
               const R *pot, int nvec, double alpha, double beta, bool fwd_next, hipStream_t st,
               hipEvent_t *ev = nullptr, const SoEpi *so = nullptr);
-// whether this grid's H.psi runs the whole-plane kernel family at prec
-bool hpsi_plane_family(const GridDev &gd, int prec);
+// whether the FP64 step takes the spin-orbit add in its epilogue (SoEpi)
+bool hpsi_so_fused(const GridDev &gd);
 
 // ---- cubic Hermite interpolation of a uniform radial table (the smooth
 // option of the differentiable path, SEP_INTERP_CUBIC).  On segment i
