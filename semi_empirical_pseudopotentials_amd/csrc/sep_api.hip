@@ -344,14 +344,16 @@ static int finish_potential(sep_ctx *c) {
   const long N = c->gd.N;
   size_t cap = 0;
   if (!c->pot32) RCHK(ensure(c, (void **)&c->pot32, &cap, sizeof(float) * N));
-  RCHK(convert_d2f(c->pot64, c->pot32, N, c->st));
-  std::vector<double> h(N);
-  HIPCHK(c, hipMemcpyAsync(h.data(), c->pot64, sizeof(double) * N, hipMemcpyDeviceToHost, c->st));
+  const long nb = finish_potential_blocks(N);
+  RCHK(ensure_scr(c, 2 * (size_t)nb));
+  RCHK(finish_potential_dev(c->pot64, c->pot32, N, c->scr, c->st));
+  std::vector<double> h(2 * nb);
+  HIPCHK(c, hipMemcpyAsync(h.data(), c->scr, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
   HIPCHK(c, hipStreamSynchronize(c->st));
   double vmin = 1.0e10, vmax = -1.0e10;  // filter/init.c:116-117,196-199
-  for (long g = 0; g < N; g++) {
-    if (vmax < h[g]) vmax = h[g];
-    if (vmin > h[g]) vmin = h[g];
+  for (long b = 0; b < nb; b++) {
+    if (vmin > h[2 * b]) vmin = h[2 * b];
+    if (vmax < h[2 * b + 1]) vmax = h[2 * b + 1];
   }
   c->vmin = vmin;
   c->vmax = vmax;

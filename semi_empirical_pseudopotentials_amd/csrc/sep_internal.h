@@ -180,6 +180,10 @@ int build_potential_dev(const GridDev &gd, double xmin, double ymin, double zmin
                         const double *scale_d, const long *npot_d, const double *vr_d,
                         const double *pot_d, long stride, const double *dr_d, double ex_e,
                         double ex_x0, double ex_t, int interp, double *potl_d, hipStream_t st);
+// FP32 copy of V and the extrema of V per workgroup: part[2 b], part[2 b + 1]
+// for b < finish_potential_blocks(n)
+long finish_potential_blocks(long n);
+int finish_potential_dev(const double *v, float *f, long n, double *part, hipStream_t st);
 // out[i] = sum_g a[i*lda + g] * b[i*ldb + g] for i < m (deterministic).
 int dots_dev(const double *a, long lda, const double *b, long ldb, long m, long n, double *out_d,
              double *scratch, long scratch_len, hipStream_t st);
