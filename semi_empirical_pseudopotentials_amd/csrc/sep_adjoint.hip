@@ -19,122 +19,166 @@
 // cubic_weights()/cubic_rows() on rows k-1 .. k+2, whose derivative in del
 // is continuous.
 //
-// Work split: one block per (atom, slice of the atom's bounding box of grid
-// points within the table range); each block reduces its partial sums over
-// the box slice in fixed order (written to a work array and summed in split
-// order by a second kernel), and accumulates its table histogram in LDS,
-// flushed with global atomic adds (so dtab is reproducible to rounding only).
+// Work split: an item is a slice of one atom's bounding box of grid points
+// within the table range; a persistent grid of two workgroups per CU takes
+// contiguous runs of items, atoms sorted by type.  An item's partial sums go
+// to a work array, summed in slice order by a second kernel.  The table
+// histogram accumulates in LDS over all of a workgroup's items of one type and
+// is flushed with global atomic adds (so dtab is reproducible to rounding
+// only).  Bound by the FP64 divisions and square root of a point, its LDS
+// atomics and the few waves that the histogram's LDS leaves on a CU (77 KB
+// for 8 pairs of 1201 rows).
 #include <hip/hip_runtime.h>
 
 #include "sep_internal.h"
 
 namespace sep {
 
-constexpr int HF_THREADS = 256;
+constexpr int HF_THREADS = 512;
+constexpr int HF_BLOCKS = 512;  // persistent workgroups: two per CU
 
+// order: atom of each item group (atoms sorted by type), items it =
+// group * nsplit + slice
 template <int PB>
-__global__ void __launch_bounds__(HF_THREADS) k_hf_atom(
+__global__ void __launch_bounds__(HF_THREADS, 4) k_hf_atom(
     int nx, int ny, int nz, double xmin, double ymin, double zmin, double dx, double dy,
     double dz, const double *__restrict__ xyz, const int *__restrict__ type,
-    const double *__restrict__ scale, const long *__restrict__ npot, const double *__restrict__ vr,
-    const double *__restrict__ pot, long stride, const double *__restrict__ dr,
-    const double *__restrict__ rho, long N, int np, int p0, int ntype, int nsplit, int interp,
-    double *__restrict__ work, double *__restrict__ htab) {
-  extern __shared__ double hist[];  // [PB][npot_t]
-  const int a = blockIdx.x, split = blockIdx.y;
-  const int t = type[a];
-  const long nt = npot[t];
-  const double drt = dr[t];
-  const double rmax = (double)(nt - 1) * drt;
-  const double Rx = xyz[3 * a], Ry = xyz[3 * a + 1], Rz = xyz[3 * a + 2];
-  const double sa = scale ? scale[a] : 1.0;
-  const double *vt = vr + t * stride, *pt = pot + t * stride;
-  for (long k = threadIdx.x; k < (long)PB * nt; k += HF_THREADS) hist[k] = 0.0;
-  __syncthreads();
-  // bounding box of grid points within rmax of the atom
-  auto lo = [](double c, double r, double o, double d) { return (int)ceil((c - r - o) / d); };
-  auto hi = [](double c, double r, double o, double d) { return (int)floor((c + r - o) / d); };
-  const int x0 = max(0, lo(Rx, rmax, xmin, dx)), x1 = min(nx - 1, hi(Rx, rmax, xmin, dx));
-  const int y0 = max(0, lo(Ry, rmax, ymin, dy)), y1 = min(ny - 1, hi(Ry, rmax, ymin, dy));
-  const int z0 = max(0, lo(Rz, rmax, zmin, dz)), z1 = min(nz - 1, hi(Rz, rmax, zmin, dz));
-  const long Lx = x1 >= x0 ? x1 - x0 + 1 : 0, Ly = y1 >= y0 ? y1 - y0 + 1 : 0,
-             Lz = z1 >= z0 ? z1 - z0 + 1 : 0;
-  const long tot = Lx * Ly * Lz;
-  const long chunk = (tot + nsplit - 1) / nsplit;
-  const long b0 = (long)split * chunk, b1 = min(tot, b0 + chunk);
-  double acc[PB][4];
-#pragma unroll
-  for (int q = 0; q < PB; q++) acc[q][0] = acc[q][1] = acc[q][2] = acc[q][3] = 0.0;
-  for (long b = b0 + threadIdx.x; b < b1; b += HF_THREADS) {
-    const int ix = x0 + (int)(b % Lx);
-    const int iy = y0 + (int)((b / Lx) % Ly);
-    const int iz = z0 + (int)(b / (Lx * Ly));
-    const double ddx = (xmin + ix * dx) - Rx, ddy = (ymin + iy * dy) - Ry,
-                 ddz = (zmin + iz * dz) - Rz;
-    const double del = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-    const long k = (long)(del / drt);
-    if (k > nt - 2) continue;
-    const double span = vt[k + 1] - vt[k];
-    const double w = (del - vt[k]) / span;
-    // value, d(value)/d(del) without the scale, and the table-row weights
-    long rows[4] = {k, k + 1, k + 1, k + 1};
-    double wr[4] = {1.0 - w, w, 0.0, 0.0};
-    double val, dval;
-    if (interp == SEP_INTERP_CUBIC) {
-      double cw[4], cd[4], dr4[4];
-      cubic_weights(w, cw, cd);
-      cubic_rows(k, nt, cw, rows, wr);
-      cubic_rows(k, nt, cd, rows, dr4);
-      val = dval = 0.0;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        val += wr[c] * pt[rows[c]];
-        dval += dr4[c] * pt[rows[c]];
-      }
-      dval /= span;
-    } else {
-      val = (1.0 - w) * pt[k] + w * pt[k + 1];
-      dval = (pt[k + 1] - pt[k]) / span;
-    }
-    const double g = del > 0.0 ? -sa * dval / del : 0.0;
-    const long gi = ((long)iz * ny + iy) * nx + ix;
-#pragma unroll
-    for (int q = 0; q < PB; q++) {
-      if (p0 + q >= np) break;
-      const double r = rho[(long)(p0 + q) * N + gi];
-      acc[q][0] += r * g * ddx;
-      acc[q][1] += r * g * ddy;
-      acc[q][2] += r * g * ddz;
-      acc[q][3] += r * val;
-#pragma unroll
-      for (int c = 0; c < 4; c++)
-        if (wr[c] != 0.0) atomicAdd(&hist[q * nt + rows[c]], r * sa * wr[c]);
-    }
-  }
-  // block reduction of the partial sums (wave shuffles, then LDS across waves)
+    const int *__restrict__ order, const double *__restrict__ scale,
+    const long *__restrict__ npot, const double *__restrict__ vr, const double *__restrict__ pot,
+    long stride, const double *__restrict__ dr, const double *__restrict__ rho, long N, int np,
+    int p0, int ntype, int nitems, int nsplit, int interp, double *__restrict__ work,
+    double *__restrict__ htab) {
+  extern __shared__ double hist[];  // [PB][npot_t] of the current type
   __shared__ double red[HF_THREADS / 64][PB * 4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < PB; q++)
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      double v = acc[q][c];
-      for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-      if (lane == 0) red[wv][q * 4 + c] = v;
+  const int it0 = (int)((long)nitems * blockIdx.x / gridDim.x);
+  const int it1 = (int)((long)nitems * (blockIdx.x + 1) / gridDim.x);
+  int cur = -1;  // type whose histogram is in LDS
+  long nt = 0;
+  // table histogram -> global (only rows the items touched are non-zero)
+  auto flush = [&]() {
+    for (int k = threadIdx.x; k < PB * (int)nt; k += HF_THREADS) {
+      const int q = k / (int)nt;
+      const double v = hist[k];
+      if (v != 0.0 && p0 + q < np)
+        atomicAdd(&htab[((long)(p0 + q) * ntype + cur) * stride + (k - q * (int)nt)], v);
     }
-  __syncthreads();
-  if (threadIdx.x < PB * 4) {
-    double v = 0.0;
-    for (int w2 = 0; w2 < HF_THREADS / 64; w2++) v += red[w2][threadIdx.x];
-    work[((long)a * nsplit + split) * PB * 4 + threadIdx.x] = v;
+  };
+  for (int it = it0; it < it1; it++) {
+    const int a = order[it / nsplit], split = it % nsplit;
+    const int t = type[a];
+    if (t != cur) {
+      if (cur >= 0) {
+        __syncthreads();
+        flush();
+        __syncthreads();
+      }
+      cur = t;
+      nt = npot[t];
+      for (int k = threadIdx.x; k < PB * (int)nt; k += HF_THREADS) hist[k] = 0.0;
+      __syncthreads();
+    }
+    const double drt = dr[t];
+    const double rmax = (double)(nt - 1) * drt;
+    const double Rx = xyz[3 * a], Ry = xyz[3 * a + 1], Rz = xyz[3 * a + 2];
+    const double sa = scale ? scale[a] : 1.0;
+    const double *vt = vr + t * stride, *pt = pot + t * stride;
+    // bounding box of grid points within rmax of the atom
+    auto lo = [](double c, double r, double o, double d) { return (int)ceil((c - r - o) / d); };
+    auto hi = [](double c, double r, double o, double d) { return (int)floor((c + r - o) / d); };
+    const int x0 = max(0, lo(Rx, rmax, xmin, dx)), x1 = min(nx - 1, hi(Rx, rmax, xmin, dx));
+    const int y0 = max(0, lo(Ry, rmax, ymin, dy)), y1 = min(ny - 1, hi(Ry, rmax, ymin, dy));
+    const int z0 = max(0, lo(Rz, rmax, zmin, dz)), z1 = min(nz - 1, hi(Rz, rmax, zmin, dz));
+    const int Lx = x1 >= x0 ? x1 - x0 + 1 : 0, Ly = y1 >= y0 ? y1 - y0 + 1 : 0,
+              Lz = z1 >= z0 ? z1 - z0 + 1 : 0;
+    const int tot = Lx * Ly * Lz;
+    const int chunk = (tot + nsplit - 1) / nsplit;
+    const int b0 = min(tot, split * chunk), b1 = min(tot, b0 + chunk);
+    double acc[PB][4];
+#pragma unroll
+    for (int q = 0; q < PB; q++) acc[q][0] = acc[q][1] = acc[q][2] = acc[q][3] = 0.0;
+    int b = b0 + threadIdx.x;
+    if (b < b1) {
+      // position in the box, advanced by the workgroup's size with carries
+      // (a division per point otherwise)
+      int ix = b % Lx, iy = b / Lx % Ly, iz = b / (Lx * Ly);
+      const int sx = HF_THREADS % Lx, sy = HF_THREADS / Lx % Ly, sz = HF_THREADS / (Lx * Ly);
+      for (; b < b1; b += HF_THREADS) {
+        const int gx = x0 + ix, gy = y0 + iy, gz = z0 + iz;
+        ix += sx;
+        iy += sy;
+        iz += sz;
+        if (ix >= Lx) {
+          ix -= Lx;
+          iy++;
+        }
+        if (iy >= Ly) {
+          iy -= Ly;
+          iz++;
+        }
+        const double ddx = (xmin + gx * dx) - Rx, ddy = (ymin + gy * dy) - Ry,
+                     ddz = (zmin + gz * dz) - Rz;
+        const double del = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
+        const long k = (long)(del / drt);
+        if (k > nt - 2) continue;
+        const double span = vt[k + 1] - vt[k];
+        const double w = (del - vt[k]) / span;
+        // value, d(value)/d(del) without the scale, and the table-row weights
+        long rows[4] = {k, k + 1, k + 1, k + 1};
+        double wr[4] = {1.0 - w, w, 0.0, 0.0};
+        double val, dval;
+        if (interp == SEP_INTERP_CUBIC) {
+          double cw[4], cd[4], dr4[4];
+          cubic_weights(w, cw, cd);
+          cubic_rows(k, nt, cw, rows, wr);
+          cubic_rows(k, nt, cd, rows, dr4);
+          val = dval = 0.0;
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            val += wr[c] * pt[rows[c]];
+            dval += dr4[c] * pt[rows[c]];
+          }
+          dval /= span;
+        } else {
+          val = (1.0 - w) * pt[k] + w * pt[k + 1];
+          dval = (pt[k + 1] - pt[k]) / span;
+        }
+        const double g = del > 0.0 ? -sa * dval / del : 0.0;
+        const long gi = ((long)gz * ny + gy) * nx + gx;
+#pragma unroll
+        for (int q = 0; q < PB; q++) {
+          if (p0 + q >= np) break;
+          const double r = rho[(long)(p0 + q) * N + gi];
+          const double rg = r * g, rs = r * sa;
+          acc[q][0] += rg * ddx;
+          acc[q][1] += rg * ddy;
+          acc[q][2] += rg * ddz;
+          acc[q][3] += r * val;
+          double *h = hist + q * (int)nt;
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+            if (wr[c] != 0.0) atomicAdd(&h[rows[c]], rs * wr[c]);
+        }
+      }
+    }
+    // partial sums of the item (wave shuffles, then LDS across waves)
+#pragma unroll
+    for (int q = 0; q < PB; q++)
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        double v = acc[q][c];
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
+        if (lane == 0) red[wv][q * 4 + c] = v;
+      }
+    __syncthreads();
+    if (threadIdx.x < PB * 4) {
+      double v = 0.0;
+      for (int w2 = 0; w2 < HF_THREADS / 64; w2++) v += red[w2][threadIdx.x];
+      work[((long)a * nsplit + split) * PB * 4 + threadIdx.x] = v;
+    }
+    __syncthreads();  // red is free for the next item
   }
-  // table histogram -> global (only rows this block touched are non-zero)
-  for (long k = threadIdx.x; k < (long)PB * nt; k += HF_THREADS) {
-    const int q = (int)(k / nt);
-    const double v = hist[k];
-    if (v != 0.0 && p0 + q < np)
-      atomicAdd(&htab[((long)(p0 + q) * ntype + t) * stride + (k - (long)q * nt)], v);
-  }
+  if (cur >= 0) flush();
 }
 
 // Sum the per-split partials in split order and scale by dv.
@@ -182,7 +226,7 @@ int pair_density_dev(const double *states, long N, const long *pairs_d, const do
 template <int PB>
 static int hf_pass(const GridDev &gd, double xmin, double ymin, double zmin, double dx, double dy,
                    double dz, double dv, int natom, const double *xyz, const int *type,
-                   const double *scale, const long *npot, long maxnpot, const double *vr,
+                   const int *order, const double *scale, const long *npot, long maxnpot, const double *vr,
                    const double *pot, long stride, const double *dr, int ntype, const double *rho,
                    int np, int p0, int nsplit, int interp, double *work, double *htab, double *dR,
                    double *dscale, hipStream_t st) {
@@ -193,51 +237,64 @@ static int hf_pass(const GridDev &gd, double xmin, double ymin, double zmin, dou
                         160 * 1024 - 4096);
     attr = true;
   }
-  hipLaunchKernelGGL(k_hf_atom<PB>, dim3((unsigned)natom, (unsigned)nsplit), dim3(HF_THREADS), lds,
-                     st, gd.nx, gd.ny, gd.nz, xmin, ymin, zmin, dx, dy, dz, xyz, type, scale, npot,
-                     vr, pot, stride, dr, rho, gd.N, np, p0, ntype, nsplit, interp, work, htab);
+  const int nitems = natom * nsplit;
+  hipLaunchKernelGGL(k_hf_atom<PB>, dim3((unsigned)(nitems < HF_BLOCKS ? nitems : HF_BLOCKS)),
+                     dim3(HF_THREADS), lds, st, gd.nx, gd.ny, gd.nz, xmin, ymin, zmin, dx, dy, dz,
+                     xyz, type, order, scale, npot, vr, pot, stride, dr, rho, gd.N, np, p0, ntype,
+                     nitems, nsplit, interp, work, htab);
   const long nthr = (long)natom * PB;
   hipLaunchKernelGGL(k_hf_reduce<PB>, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st, work,
                      natom, nsplit, np, p0, dv, dR, dscale);
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
-// Largest pair batch whose LDS histogram (PB x maxnpot doubles) fits 152 KB.
-int hf_pairs_per_pass(long maxnpot) {
+// Slices per atom: enough items for the persistent grid to balance (four per
+// workgroup), none below 1024 points of a box of `box` points.
+int hf_slices(long natom, double box) {
+  long n = (4L * HF_BLOCKS + natom - 1) / natom;
+  const long most = (long)(box / 1024.0) + 1;
+  if (n > most) n = most;
+  return (int)(n > 64 ? 64 : n);
+}
+
+// Pairs of one pass: the largest batch whose LDS histogram (pairs x maxnpot
+// doubles) fits 152 KB, no larger than np needs (a single density would pay
+// the registers and LDS of eight); 0 if one does not fit.
+int hf_pairs_per_pass(long maxnpot, long np) {
   const long cap = (160 * 1024 - 8192) / 8;
-  for (int pb = 8; pb > 1; pb /= 2)
-    if ((long)pb * maxnpot <= cap) return pb;
-  return maxnpot <= cap ? 1 : 0;
+  int pb = 8;
+  while (pb > 1 && ((long)pb * maxnpot > cap || pb / 2 >= np)) pb /= 2;
+  return (long)pb * maxnpot <= cap ? pb : 0;
 }
 
 int hf_adjoint_dev(const GridDev &gd, double xmin, double ymin, double zmin, double dx, double dy,
                    double dz, double dv, int natom, const double *xyz, const int *type,
-                   const double *scale, const long *npot, long maxnpot, const double *vr,
+                   const int *order, const double *scale, const long *npot, long maxnpot, const double *vr,
                    const double *pot, long stride, const double *dr, int ntype, const double *rho,
                    int np, int nsplit, int interp, double *work, double *htab, double *dR,
                    double *dscale, hipStream_t st) {
-  const int pb = hf_pairs_per_pass(maxnpot);
+  const int pb = hf_pairs_per_pass(maxnpot, np);
   if (pb == 0) return SEP_ERR_ARG;
   for (int p0 = 0; p0 < np; p0 += pb) {
     int rc;
     switch (pb) {
       case 8:
-        rc = hf_pass<8>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, scale, npot,
+        rc = hf_pass<8>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, order, scale, npot,
                         maxnpot, vr, pot, stride, dr, ntype, rho, np, p0, nsplit, interp, work, htab,
                         dR, dscale, st);
         break;
       case 4:
-        rc = hf_pass<4>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, scale, npot,
+        rc = hf_pass<4>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, order, scale, npot,
                         maxnpot, vr, pot, stride, dr, ntype, rho, np, p0, nsplit, interp, work, htab,
                         dR, dscale, st);
         break;
       case 2:
-        rc = hf_pass<2>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, scale, npot,
+        rc = hf_pass<2>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, order, scale, npot,
                         maxnpot, vr, pot, stride, dr, ntype, rho, np, p0, nsplit, interp, work, htab,
                         dR, dscale, st);
         break;
       default:
-        rc = hf_pass<1>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, scale, npot,
+        rc = hf_pass<1>(gd, xmin, ymin, zmin, dx, dy, dz, dv, natom, xyz, type, order, scale, npot,
                         maxnpot, vr, pot, stride, dr, ntype, rho, np, p0, nsplit, interp, work, htab,
                         dR, dscale, st);
     }

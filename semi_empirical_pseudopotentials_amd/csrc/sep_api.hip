@@ -1899,20 +1899,22 @@ extern "C" int sep_hf_adjoint(sep_ctx *c, long npairs, const long *pairs, const 
       return fail(c, SEP_ERR_ARG, "atom %ld: bad type or table", a);
     if (npot[type[a]] > maxnpot) maxnpot = npot[type[a]];
   }
-  if (hf_pairs_per_pass(maxnpot) == 0)
+  if (hf_pairs_per_pass(maxnpot, 1) == 0)
     return fail(c, SEP_ERR_ARG, "tables of %ld rows exceed the LDS histogram", maxnpot);
   HIPCHK(c, hipSetDevice(c->device));
   const long N = c->gd.N;
   const long np = weights ? 1 : npairs;
-  // box points per atom -> slices per atom (>= ~4096 points per block)
+  // box points per atom -> slices per atom
   double rmax = 0.0;
   for (int t = 0; t < ntype; t++)
     if (npot[t] >= 2 && (double)(npot[t] - 1) * dr[t] > rmax) rmax = (double)(npot[t] - 1) * dr[t];
   const double box = (2.0 * rmax / c->dx + 1.0) * (2.0 * rmax / c->dy + 1.0) * (2.0 * rmax / c->dz + 1.0);
-  long nsplit = (long)(box / 4096.0) + 1;
-  if (nsplit > 64) nsplit = 64;
-  const int pb = hf_pairs_per_pass(maxnpot);
-  DevBuf xyz_d, type_d, npot_d, vr_d, pot_d, dr_d, scale_d, pairs_d, w_d, rho_d, work_d, htab_d,
+  const long nsplit = hf_slices(natom, box);
+  std::vector<int> order(natom);  // atoms by type, so that a table's histogram stays in LDS
+  for (long i = 0; i < natom; i++) order[i] = (int)i;
+  std::stable_sort(order.begin(), order.end(), [type](int x, int y) { return type[x] < type[y]; });
+  const int pb = hf_pairs_per_pass(maxnpot, np);
+  DevBuf xyz_d, type_d, order_d, npot_d, vr_d, pot_d, dr_d, scale_d, pairs_d, w_d, rho_d, work_d, htab_d,
       dR_d, ds_d;
   RCHK(dev_upload(c, xyz_d, xyz, sizeof(double) * 3 * natom));
   RCHK(dev_upload(c, type_d, type, sizeof(int) * natom));
@@ -1921,6 +1923,7 @@ extern "C" int sep_hf_adjoint(sep_ctx *c, long npairs, const long *pairs, const 
   RCHK(dev_upload(c, pot_d, pot, sizeof(double) * ntype * stride));
   RCHK(dev_upload(c, dr_d, dr, sizeof(double) * ntype));
   if (scale) RCHK(dev_upload(c, scale_d, scale, sizeof(double) * natom));
+  RCHK(dev_upload(c, order_d, order.data(), sizeof(int) * natom));
   RCHK(dev_upload(c, pairs_d, pairs, sizeof(long) * 2 * npairs));
   if (weights) RCHK(dev_upload(c, w_d, weights, sizeof(double) * npairs));
   RCHK(dev_alloc(c, rho_d, sizeof(double) * np * N));
@@ -1932,8 +1935,8 @@ extern "C" int sep_hf_adjoint(sep_ctx *c, long npairs, const long *pairs, const 
   RCHK(pair_density_dev(c->states, N, pairs_d.as<long>(), w_d.as<double>(), (int)npairs,
                         rho_d.as<double>(), c->st));
   int rc = hf_adjoint_dev(c->gd, c->xmin, c->ymin, c->zmin, c->dx, c->dy, c->dz, c->dv, (int)natom,
-                          xyz_d.as<double>(), type_d.as<int>(), scale_d.as<double>(),
-                          npot_d.as<long>(), maxnpot, vr_d.as<double>(), pot_d.as<double>(), stride,
+                          xyz_d.as<double>(), type_d.as<int>(), order_d.as<int>(),
+                          scale_d.as<double>(), npot_d.as<long>(), maxnpot, vr_d.as<double>(), pot_d.as<double>(), stride,
                           dr_d.as<double>(), ntype, rho_d.as<double>(), (int)np, (int)nsplit,
                           c->interp, work_d.as<double>(), htab_d.as<double>(), dR_d.as<double>(),
                           ds_d.as<double>(), c->st);
