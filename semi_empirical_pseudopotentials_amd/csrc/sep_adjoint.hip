@@ -27,7 +27,10 @@
 // is flushed with global atomic adds (so dtab is reproducible to rounding
 // only).  Bound by the FP64 divisions and square root of a point, its LDS
 // atomics and the few waves that the histogram's LDS leaves on a CU (77 KB
-// for 8 pairs of 1201 rows).
+// for 8 pairs of 1201 rows).  693 atoms on 96^3, linear tables: one density
+// 186 us (539 with a workgroup per slice), 3 pairs 251 (730), 8 pairs 430
+// (1179; 748 before the row weights were specialised by interpolation and the
+// densities loaded ahead of the geometry).
 #include <hip/hip_runtime.h>
 
 #include "sep_internal.h"
@@ -39,14 +42,14 @@ constexpr int HF_BLOCKS = 512;  // persistent workgroups: two per CU
 
 // order: atom of each item group (atoms sorted by type), items it =
 // group * nsplit + slice
-template <int PB>
+template <int PB, bool CUBIC>
 __global__ void __launch_bounds__(HF_THREADS, 4) k_hf_atom(
     int nx, int ny, int nz, double xmin, double ymin, double zmin, double dx, double dy,
     double dz, const double *__restrict__ xyz, const int *__restrict__ type,
     const int *__restrict__ order, const double *__restrict__ scale,
     const long *__restrict__ npot, const double *__restrict__ vr, const double *__restrict__ pot,
     long stride, const double *__restrict__ dr, const double *__restrict__ rho, long N, int np,
-    int p0, int ntype, int nitems, int nsplit, int interp, double *__restrict__ work,
+    int p0, int ntype, int nitems, int nsplit, double *__restrict__ work,
     double *__restrict__ htab) {
   extern __shared__ double hist[];  // [PB][npot_t] of the current type
   __shared__ double red[HF_THREADS / 64][PB * 4];
@@ -119,45 +122,66 @@ __global__ void __launch_bounds__(HF_THREADS, 4) k_hf_atom(
         const double ddx = (xmin + gx * dx) - Rx, ddy = (ymin + gy * dy) - Ry,
                      ddz = (zmin + gz * dz) - Rz;
         const double del = sqrt(ddx * ddx + ddy * ddy + ddz * ddz);
-        const long k = (long)(del / drt);
-        if (k > nt - 2) continue;
-        const double span = vt[k + 1] - vt[k];
-        const double w = (del - vt[k]) / span;
-        // value, d(value)/d(del) without the scale, and the table-row weights
-        long rows[4] = {k, k + 1, k + 1, k + 1};
-        double wr[4] = {1.0 - w, w, 0.0, 0.0};
+        const long kl = (long)(del / drt);
+        if (kl > nt - 2) continue;
+        const int k = (int)kl;
+        // the pairs' densities first, in flight under the geometry (loads
+        // between the LDS atomics would each wait for the one before)
+        const unsigned go = (unsigned)((gz * ny + gy) * nx + gx) * (unsigned)sizeof(double);
+        double rq[PB];
+#pragma unroll
+        for (int q = 0; q < PB; q++)
+          rq[q] = p0 + q < np ? *reinterpret_cast<const double *>(
+                                    reinterpret_cast<const char *>(rho + (long)(p0 + q) * N) + go)
+                              : 0.0;
+        const double v0 = vt[k];
+        const double span = vt[k + 1] - v0;
+        const double w = (del - v0) / span;
+        // value, d(value)/d(del) without the scale, and the table-row weights:
+        // rows k, k + 1 (linear), or four rows (cubic)
+        constexpr int NR = CUBIC ? 4 : 2;
+        int rows[NR];
+        double wr[NR];
         double val, dval;
-        if (interp == SEP_INTERP_CUBIC) {
+        if constexpr (CUBIC) {
           double cw[4], cd[4], dr4[4];
+          long r4[4];
           cubic_weights(w, cw, cd);
-          cubic_rows(k, nt, cw, rows, wr);
-          cubic_rows(k, nt, cd, rows, dr4);
+          cubic_rows(k, nt, cw, r4, wr);
+          cubic_rows(k, nt, cd, r4, dr4);
           val = dval = 0.0;
 #pragma unroll
           for (int c = 0; c < 4; c++) {
+            rows[c] = (int)r4[c];
             val += wr[c] * pt[rows[c]];
             dval += dr4[c] * pt[rows[c]];
           }
           dval /= span;
         } else {
-          val = (1.0 - w) * pt[k] + w * pt[k + 1];
-          dval = (pt[k + 1] - pt[k]) / span;
+          rows[0] = k;
+          rows[1] = k + 1;
+          wr[0] = 1.0 - w;
+          wr[1] = w;
+          const double pa = pt[k], pb = pt[k + 1];
+          val = wr[0] * pa + w * pb;
+          dval = (pb - pa) / span;
         }
         const double g = del > 0.0 ? -sa * dval / del : 0.0;
-        const long gi = ((long)gz * ny + gy) * nx + gx;
+        const double fx = g * ddx, fy = g * ddy, fz = g * ddz;
+#pragma unroll
+        for (int c = 0; c < NR; c++) wr[c] *= sa;
 #pragma unroll
         for (int q = 0; q < PB; q++) {
           if (p0 + q >= np) break;
-          const double r = rho[(long)(p0 + q) * N + gi];
-          const double rg = r * g, rs = r * sa;
-          acc[q][0] += rg * ddx;
-          acc[q][1] += rg * ddy;
-          acc[q][2] += rg * ddz;
+          const double r = rq[q];
+          acc[q][0] += r * fx;
+          acc[q][1] += r * fy;
+          acc[q][2] += r * fz;
           acc[q][3] += r * val;
           double *h = hist + q * (int)nt;
 #pragma unroll
-          for (int c = 0; c < 4; c++)
-            if (wr[c] != 0.0) atomicAdd(&h[rows[c]], rs * wr[c]);
+          for (int c = 0; c < NR; c++)
+            if (wr[c] != 0.0) atomicAdd(&h[rows[c]], r * wr[c]);
         }
       }
     }
@@ -231,17 +255,23 @@ static int hf_pass(const GridDev &gd, double xmin, double ymin, double zmin, dou
                    int np, int p0, int nsplit, int interp, double *work, double *htab, double *dR,
                    double *dscale, hipStream_t st) {
   const size_t lds = sizeof(double) * PB * (size_t)maxnpot;
-  static bool attr = false;
-  if (!attr) {
-    hipFuncSetAttribute((const void *)k_hf_atom<PB>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                        160 * 1024 - 4096);
-    attr = true;
-  }
   const int nitems = natom * nsplit;
-  hipLaunchKernelGGL(k_hf_atom<PB>, dim3((unsigned)(nitems < HF_BLOCKS ? nitems : HF_BLOCKS)),
-                     dim3(HF_THREADS), lds, st, gd.nx, gd.ny, gd.nz, xmin, ymin, zmin, dx, dy, dz,
-                     xyz, type, order, scale, npot, vr, pot, stride, dr, rho, gd.N, np, p0, ntype,
-                     nitems, nsplit, interp, work, htab);
+  auto launch = [&](auto *kernel, bool *attr) {
+    if (!*attr) {
+      hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          160 * 1024 - 4096);
+      *attr = true;
+    }
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(nitems < HF_BLOCKS ? nitems : HF_BLOCKS)),
+                       dim3(HF_THREADS), lds, st, gd.nx, gd.ny, gd.nz, xmin, ymin, zmin, dx, dy, dz,
+                       xyz, type, order, scale, npot, vr, pot, stride, dr, rho, gd.N, np, p0, ntype,
+                       nitems, nsplit, work, htab);
+  };
+  static bool attr[2] = {false, false};
+  if (interp == SEP_INTERP_CUBIC)
+    launch(k_hf_atom<PB, true>, &attr[1]);
+  else
+    launch(k_hf_atom<PB, false>, &attr[0]);
   const long nthr = (long)natom * PB;
   hipLaunchKernelGGL(k_hf_reduce<PB>, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, st, work,
                      natom, nsplit, np, p0, dv, dR, dscale);
