@@ -68,6 +68,9 @@ struct sep_ctx {
   // spin-orbit lists of the spinor H (sep_so_setup) and the per-entry
   // contributions of one application
   SoLists so;
+  // pinned staging of large downloads (two halves), created on first use
+  char *stage = nullptr;
+  hipEvent_t sev[2] = {};
   double *so_contrib = nullptr;
   size_t so_contrib_bytes = 0;
   std::string err;
@@ -166,6 +169,51 @@ static int ensure_scr(sep_ctx *c, size_t len) {
   size_t cap = c->scr_len * sizeof(double);
   RCHK(ensure(c, (void **)&c->scr, &cap, len * sizeof(double)));
   if (len > c->scr_len) c->scr_len = len;
+  return SEP_OK;
+}
+
+// Device -> host copy, complete on return (after the work queued on st).
+// Large ones go through two pinned halves, the GPU filling one while up to
+// eight threads copy the other out: a fresh destination's page faults and
+// clearing cost a single-threaded copy more than the transfer itself (268 MB
+// to fresh memory: hipMemcpy 26.6 ms, staged 5.9 ms with 8 MB halves, 8.0 ms
+// with 4 MB ones).  Below STAGE_MIN the plain copy is as fast.
+static constexpr size_t STAGE_HALF = 8u << 20, STAGE_MIN = 8u << 20;
+static int download(sep_ctx *c, void *dst, const void *src, size_t bytes) {
+  if (bytes >= STAGE_MIN && !c->stage) {
+    if (hipHostMalloc((void **)&c->stage, 2 * STAGE_HALF, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      c->stage = nullptr;
+    }
+    for (hipEvent_t &e : c->sev)
+      if (c->stage && !e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        e = nullptr;
+        hipHostFree(c->stage);
+        c->stage = nullptr;
+      }
+  }
+  if (bytes < STAGE_MIN || !c->stage) {
+    HIPCHK(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    return SEP_OK;
+  }
+  // eight pieces at least, so that the first and the last cost little
+  const size_t piece = std::min(STAGE_HALF, (bytes / 8 + 4095) / 4096 * 4096);
+  const size_t n = (bytes + piece - 1) / piece;
+  for (size_t i = 0; i <= n; i++) {
+    if (i < n) {
+      HIPCHK(c, hipMemcpyAsync(c->stage + (i & 1) * STAGE_HALF, (const char *)src + i * piece,
+                               std::min(piece, bytes - i * piece), hipMemcpyDeviceToHost, c->st));
+      HIPCHK(c, hipEventRecord(c->sev[i & 1], c->st));
+    }
+    if (i > 0) {
+      const size_t k = i - 1;
+      HIPCHK(c, hipEventSynchronize(c->sev[k & 1]));
+      sep_par_copy((char *)dst + k * piece, c->stage + (k & 1) * STAGE_HALF,
+                   std::min(piece, bytes - k * piece));
+    }
+  }
   return SEP_OK;
 }
 
@@ -330,6 +378,9 @@ int sep_close(sep_ctx *c) {
   if (c->blas) rocblas_destroy_handle(c->blas);
   if (c->dws) hipFree(c->dws);
   if (c->zpot) hipFree(c->zpot);
+  if (c->stage) hipHostFree(c->stage);
+  for (hipEvent_t e : c->sev)
+    if (e) hipEventDestroy(e);
   for (hipStream_t s : c->lst)
     if (s) hipStreamDestroy(s);
   for (hipEvent_t e : c->lev)
@@ -406,8 +457,7 @@ int sep_build_potential(sep_ctx *c, long natom, const double *xyz, const int *ty
   HIPCHK(c, hipStreamSynchronize(c->st));
   if (rc != SEP_OK) return fail(c, rc, "potential kernel launch failed");
   RCHK(finish_potential(c));
-  if (potl_out)
-    HIPCHK(c, hipMemcpy(potl_out, c->pot64, sizeof(double) * N, hipMemcpyDeviceToHost));
+  if (potl_out) RCHK(download(c, potl_out, c->pot64, sizeof(double) * N));
   if (vmin) *vmin = c->vmin;
   if (vmax) *vmax = c->vmax;
   return SEP_OK;
@@ -536,7 +586,7 @@ int sep_hnorm(sep_ctx *c, const double *in, double *out, long batch, double zm1,
     VecView<double> v{nullptr, nullptr, p, N};
     rc = apply_views<double>(c, v, v, (int)nb, alpha, beta, nullptr);
   }
-  if (rc == SEP_OK && hipMemcpy(out, d, bytes, hipMemcpyDeviceToHost) != hipSuccess) rc = SEP_ERR_HIP;
+  if (rc == SEP_OK) rc = download(c, out, d, bytes);
   hipFree(d);
   if (rc == SEP_ERR_HIP) return fail(c, rc, "hnorm: HIP copy failed");
   return rc;
@@ -693,9 +743,7 @@ int sep_states_upload(sep_ctx *c, const double *psi, long m) {
 int sep_states_download(sep_ctx *c, double *psi, long m) {
   if (!c || !psi || m < 1 || m > c->cap1) return SEP_ERR_ARG;
   HIPCHK(c, hipSetDevice(c->device));
-  HIPCHK(c, hipStreamSynchronize(c->st));
-  HIPCHK(c, hipMemcpy(psi, c->states, sizeof(double) * m * c->gd.N, hipMemcpyDeviceToHost));
-  return SEP_OK;
+  return download(c, psi, c->states, sizeof(double) * m * c->gd.N);
 }
 int sep_normalize_all(sep_ctx *c, long m) {
   if (!c || m < 0 || m > c->cap1) return SEP_ERR_ARG;
@@ -2346,6 +2394,8 @@ extern "C" int sep_trim(sep_ctx *c) {
   if (c->gwork) HIPCHK(c, hipFree(c->gwork));
   c->gwork = nullptr;
   c->gwork_bytes = 0;
+  if (c->stage) HIPCHK(c, hipHostFree(c->stage));
+  c->stage = nullptr;
   return SEP_OK;
 }
 

@@ -17,6 +17,19 @@
 #include "../../include/sep_deck.h"
 #include "sep_host.h"
 
+void sep_par_copy(void *dst, const void *src, size_t n) {
+  enum { PARTS = 8 };
+  if (n < (1 << 20)) {
+    memcpy(dst, src, n);
+    return;
+  }
+#pragma omp parallel for schedule(static) num_threads(PARTS)
+  for (int p = 0; p < PARTS; p++) {
+    const size_t a = n / PARTS * p, b = p + 1 < PARTS ? n / PARTS * (p + 1) : n;
+    memcpy((char *)dst + a, (const char *)src + a, b - a);
+  }
+}
+
 /* ===================================================== random numbers */
 /* L'Ecuyer two-generator combination with a 32-entry Bays-Durham shuffle;
  * constants as filter/rand.c:11-24. */
