@@ -165,79 +165,100 @@ __global__ void __launch_bounds__(SO_T) k_so_kmat(SoLists so) {
   }
 }
 
-// k_so_contrib with K read from the matrices of k_so_kmat: KT threads, NP
-// points p per thread.  A 1-D grid over ceil(natom / 8) * 8 * nsp blocks:
-// block b runs on XCD b % 8 (round-robin dispatch), and the blocks of one
-// atom share that XCD and sit close in the dispatch order, so the atom's K
-// is read from HBM once and from that XCD's L2 by its other spinors.
-// Measured at 96^3 with 465 atoms (244-277 points each), 8 spinors: KT =
-// 256, NP = 1 209 us per call (26 TFLOP/s FP64); KT = 128, NP = 2 (half the
-// LDS bytes per FMA) 348 us; one wave per spinor with four spinors at 64
-// shared points per workgroup (K from L2 a quarter as often) 216 us; the
-// 12 products per q written to memory first (44 us) and read back at
-// wave-uniform addresses through scalar loads, with no LDS (62 VGPRs,
-// occupancy 8) 246 us; K of the next 8 q's loaded while the current 8 are
-// consumed 199 against 208 us (not kept: no gain in the filter's time) --
-// neither the LDS bytes per FMA nor the L2 stream of K sets its pace.  Each
-// point's sums run over q in the order of k_so_contrib: the two kernels
-// agree bit for bit.
-template <int KT, int NP>
-__global__ void __launch_bounds__(KT) k_so_contrib_k(SoLists so, const double *in, long cs,
-                                                     long ss, double *contrib, long nsp) {
-  const long b = blockIdx.x;
-  const long x = b % 8, j = b / 8;
-  const long s = j % nsp, a = (j / nsp) * 8 + x;
-  if (a >= so.natom) return;  // padding blocks of the last group of eight
-  const long o0 = so.off[a], n = so.off[a + 1] - o0;
+// k_so_contrib with K read from the matrices of k_so_kmat, as a register-tiled
+// product: S[p][spinor, 12] = sum_q K(q, p) w(q)[spinor, 12].  A workgroup
+// takes 32 PT points p of one atom and up to SB spinors, half a wave per
+// spinor, PT points per lane: a K read from LDS serves 12 multiply-adds, a w
+// PT.  K rows and the point densities of the next SO_QK q's are loaded into
+// registers while the current ones are consumed: without that the latency of
+// the K stream sets the pace (8 spinors or 1 take the same 430 us).  Bound by
+// the LDS reads, 12 + PT words a lane for 12 PT multiply-adds.  465 atoms of 244-277
+// points at 96^3 (8 spinors: 5.5 GFLOP FP64, 85 us at the VALU's rate), in us
+// at 8 / 4 / 2 / 1 spinors: one point a lane and K from L2 273 / 161 / 115 /
+// 105, now 192 / 129 / 102 / 96.  K on the matrix cores would not help: their
+// FP64 rate is below the VALU's here (sep_gemm.hip).  Skipping the 32-point
+// rows past the list by a branch stops the LDS reads from running ahead (293).
+// Workgroup b runs on XCD b % 8; an atom's workgroups share that XCD.  Each
+// point's sums run over q in the order of k_so_contrib: bit for bit the same.
+static constexpr int SO_QK = 32;  // q points per LDS tile
+template <int PT, int SB>
+__global__ void __launch_bounds__(32 * SB, 2)
+    k_so_contrib_k(SoLists so, const double *in, long cs, long ss, double *contrib, int nsp, int sb,
+                   int ngrp, int npt) {
+  constexpr int T = 32 * SB, PB = 32 * PT, NK = SO_QK * PB / T;
+  static_assert(SO_QK * SB == T, "one product set per thread and tile");
+  const int b = blockIdx.x;
+  int jg = b / 8;
+  const int ip = jg % npt;
+  jg /= npt;
+  const int s0 = jg % ngrp * sb, a = jg / ngrp * 8 + b % 8;
+  if (a >= so.natom) return;  // padding workgroups of the last eight atoms
+  const long o0 = so.off[a];
+  const int n = (int)(so.off[a + 1] - o0);
+  const int p0 = ip * PB;
+  if (p0 >= n) return;
+  const int ns = min(sb, nsp - s0);
   const double *km = so.kmat + so.koff[a];
-  const double *ps = in + s * ss;
-  __shared__ __align__(16) double qw[SO_QT][12];
-  const double c = so.c;
-  for (long p0 = 0; p0 < n; p0 += KT * NP) {
-    // points past the list read row entries of the last point (in bounds)
-    // and are not written
-    long pc[NP];
+  __shared__ __align__(16) double qw[SO_QK][SB][12];
+  __shared__ __align__(16) double qk[SO_QK][PB];
+  const int t = threadIdx.x;
+  const int sl = t / 32, lp = t % 32;
+  // next tile: K rows (points past the list read the last one's, rows past it
+  // the last row: in bounds and unused), and one point of one spinor
+  double kn[NK], gn[9], un[4];
+  const int tq = t % SO_QK, ts = t / SO_QK;
+  const double *ps = in + (s0 + min(ts, ns - 1)) * ss;
+  auto fetch = [&](int q0) {
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-      const long p = p0 + threadIdx.x + i * KT;
-      pc[i] = p < n ? p : n - 1;
+    for (int i = 0; i < NK; i++) {
+      const int e = t + T * i;
+      kn[i] = km[(long)min(q0 + e / PB, n - 1) * n + min(p0 + e % PB, n - 1)];
     }
-    double S[NP][12];
+    const long q = o0 + min(q0 + tq, n - 1);
+    const long jq = so.jxyz[q];
 #pragma unroll
-    for (int i = 0; i < NP; i++)
+    for (int k = 0; k < 9; k++) gn[k] = so.geo[q * 9 + k];
 #pragma unroll
-      for (int k = 0; k < 12; k++) S[i][k] = 0.0;
-    for (long q0 = 0; q0 < n; q0 += SO_QT) {
-      __syncthreads();  // the previous tile is consumed
-      for (int t = threadIdx.x; t < SO_QT; t += KT) {
-        const long q = q0 + t;
-        if (q < n) {
-          const double *g = so.geo + (o0 + q) * 9;
-          const long jq = so.jxyz[o0 + q];
-          so_point_w(g, ps[jq], ps[cs + jq], ps[2 * cs + jq], ps[3 * cs + jq], qw[t]);
-        }
-      }
-      __syncthreads();
-      const int qn = (int)(n - q0 < SO_QT ? n - q0 : SO_QT);
-      const double *kq = km + q0 * n;
-#pragma unroll 4
-      for (int t = 0; t < qn; t++) {
-        double K[NP];
+    for (int k = 0; k < 4; k++) un[k] = ps[k * cs + jq];
+  };
+  double S[PT][12];
 #pragma unroll
-        for (int i = 0; i < NP; i++) K[i] = kq[t * n + pc[i]];
+  for (int i = 0; i < PT; i++)
+#pragma unroll
+    for (int k = 0; k < 12; k++) S[i][k] = 0.0;
+  fetch(0);
+  for (int q0 = 0; q0 < n; q0 += SO_QK) {
+    __syncthreads();  // the previous tile is consumed
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+      const int e = t + T * i;
+      qk[e / PB][e % PB] = kn[i];
+    }
+    so_point_w(gn, un[0], un[1], un[2], un[3], qw[tq][ts]);
+    __syncthreads();
+    if (q0 + SO_QK < n) fetch(q0 + SO_QK);
+    const int qn = min(SO_QK, n - q0);
+    if (sl < ns) {
+#pragma unroll 2
+      for (int q = 0; q < qn; q++) {
         double w[12];
 #pragma unroll
-        for (int k = 0; k < 12; k++) w[k] = qw[t][k];
+        for (int k = 0; k < 12; k++) w[k] = qw[q][sl][k];
 #pragma unroll
-        for (int i = 0; i < NP; i++)
+        for (int i = 0; i < PT; i++) {
+          const double K = qk[q][lp + 32 * i];
 #pragma unroll
-          for (int k = 0; k < 12; k++) S[i][k] = fma(K[i], w[k], S[i][k]);
+          for (int k = 0; k < 12; k++) S[i][k] = fma(K, w[k], S[i][k]);
+        }
       }
     }
+  }
+  if (sl < ns) {
 #pragma unroll
-    for (int i = 0; i < NP; i++) {
-      const long p = p0 + threadIdx.x + i * KT;
-      if (p < n) so_point_out(so.geo + (o0 + p) * 9, c, S[i], contrib + ((o0 + p) * nsp + s) * 4);
+    for (int i = 0; i < PT; i++) {
+      const int p = p0 + lp + i * 32;
+      if (p < n)
+        so_point_out(so.geo + (o0 + p) * 9, so.c, S[i], contrib + ((o0 + p) * nsp + s0 + sl) * 4);
     }
   }
 }
@@ -310,9 +331,25 @@ int so_kmat_build(SoLists &so, const std::vector<long> &off, hipStream_t st) {
 static void so_contrib_launch(const SoLists &so, const double *in, long cs, long ss, long nsp,
                               double *contrib, hipStream_t st) {
   if (so.kmat) {
-    const long nb = (long)((so.natom + 7) / 8) * 8 * nsp;
-    hipLaunchKernelGGL((k_so_contrib_k<256, 1>), dim3((unsigned)nb), dim3(256), 0, st, so, in, cs,
-                       ss, contrib, nsp);
+    auto launch = [&](auto *kernel, int pb, int most) {
+      const int ngrp = (int)((nsp + most - 1) / most), sb = (int)((nsp + ngrp - 1) / ngrp);
+      const int npt = (int)((so.maxn + pb - 1) / pb);
+      hipLaunchKernelGGL(kernel, dim3((unsigned)((so.natom + 7) / 8 * 8 * ngrp * npt)),
+                         dim3(32 * most), 0, st, so, in, cs, ss, contrib, (int)nsp, sb, ngrp, npt);
+    };
+    // more points a lane as long as the workgroups fill the chip: 8 spinors
+    // at 128 / 64 points a workgroup 192 / 215 us with 465 atoms (1395
+    // workgroups at 128), 62 / 46 with 140 (420); 3 spinors at 64 / 32 points
+    // 18 / 16 us with 36 atoms (180 workgroups at 64)
+    const auto groups = [&](long pb) { return so.natom * ((so.maxn + pb - 1) / pb); };
+    if (nsp > 4 && groups(128) * ((nsp + 7) / 8) >= 1024)
+      launch(k_so_contrib_k<4, 8>, 128, 8);
+    else if (nsp > 4)
+      launch(k_so_contrib_k<2, 8>, 64, 8);
+    else if (groups(64) >= 256)
+      launch(k_so_contrib_k<2, 4>, 64, 4);
+    else
+      launch(k_so_contrib_k<1, 4>, 32, 4);
   } else {
     hipLaunchKernelGGL(k_so_contrib, dim3((unsigned)so.natom, (unsigned)nsp), dim3(SO_T), 0, st,
                        so, in, cs, ss, contrib, nsp);
