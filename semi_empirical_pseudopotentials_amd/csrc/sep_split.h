@@ -96,25 +96,29 @@ __device__ __forceinline__ void dft_x(cx<R> *v) {
 // j + k B, outputs A j + k), exchange, radix B on j < A (inputs and outputs
 // j + k A, twiddles w_N^(j k)).  Inverse: the same backwards (radix B, then
 // A), so that its first pass reads the registers the forward one ended with.
-// GZ threads share a z line.
+// GZ threads share a z line: as many as leave few of them idle in either pass
+// and few points a thread; at 160 ten keep 20 points a thread, which fit FP32's
+// registers (16 threads: 80 -> 98 us, 4 vectors) but not FP64's (166 -> 180).
+// At 80 ten for eight 33.2 -> 31.7 us FP64, 21.9 -> 20.7 FP32 (8 vectors).
 template <int N>
 struct LinePlan;
-#define SEP_LINE_PLAN(N_, A_, B_, GZ_)                        \
+#define SEP_LINE_PLAN(N_, A_, B_, GZ64_, GZ32_)               \
   template <>                                                 \
   struct LinePlan<N_> {                                       \
-    static constexpr int N = N_, A = A_, B = B_, GZ = GZ_;    \
+    static constexpr int N = N_, A = A_, B = B_;              \
+    static constexpr int GZ64 = GZ64_, GZ32 = GZ32_;          \
     static_assert(A_ * B_ == N_, "two-pass plan");            \
   };
-SEP_LINE_PLAN(16, 4, 4, 4)
-SEP_LINE_PLAN(24, 6, 4, 4)
-SEP_LINE_PLAN(32, 8, 4, 4)
-SEP_LINE_PLAN(36, 6, 6, 6)
-SEP_LINE_PLAN(48, 6, 8, 8)
-SEP_LINE_PLAN(64, 8, 8, 8)
-SEP_LINE_PLAN(80, 10, 8, 8)
-SEP_LINE_PLAN(96, 16, 6, 8)
-SEP_LINE_PLAN(128, 16, 8, 8)
-SEP_LINE_PLAN(160, 16, 10, 10)
+SEP_LINE_PLAN(16, 4, 4, 4, 4)
+SEP_LINE_PLAN(24, 6, 4, 4, 4)
+SEP_LINE_PLAN(32, 8, 4, 4, 4)
+SEP_LINE_PLAN(36, 6, 6, 6, 6)
+SEP_LINE_PLAN(48, 6, 8, 8, 8)
+SEP_LINE_PLAN(64, 8, 8, 8, 8)
+SEP_LINE_PLAN(80, 10, 8, 10, 10)
+SEP_LINE_PLAN(96, 16, 6, 8, 8)
+SEP_LINE_PLAN(128, 16, 8, 8, 8)
+SEP_LINE_PLAN(160, 16, 10, 16, 10)
 #undef SEP_LINE_PLAN
 
 // y lines: AY rows per group of k_xrows (register-local pass), BY points per
@@ -482,7 +486,7 @@ k_xrows_bwd(cx<R> *tb, VecView<R> pin, VecView<R> out, Epi<R> epi, int npair, in
 template <typename R, int BY, int W, int NZ>
 struct TileCfg {
   using PZ = LinePlan<NZ>;
-  static constexpr int G = PZ::GZ, A = PZ::A, B = PZ::B;
+  static constexpr int G = sizeof(R) == 8 ? PZ::GZ64 : PZ::GZ32, A = PZ::A, B = PZ::B;
   static constexpr int L = W * BY;  // z lines of the tile
   static constexpr int T = L * G;
   static_assert(T % (2 * W) == 0, "whole runs of T");
@@ -490,15 +494,19 @@ struct TileCfg {
   static constexpr int RY = (W * NZ + T - 1) / T;  // y butterflies per thread
   static constexpr int E0 = NB0 * A > NB1 * B ? NB0 * A : NB1 * B;
   static constexpr int E = E0 > RY * BY ? E0 : RY * BY;
-  // pitch of a z row in LDS: at least L, and congruent to W modulo the
-  // elements that one cycle of the LDS serves, so that the W-element runs of
-  // consecutive z fall on different banks
+  // pitch of a z row in LDS: at least L, and an odd multiple of W modulo the
+  // elements that one cycle of the LDS serves (W itself where W does not divide
+  // them), so that the W-element runs of consecutive z fall on different banks
   static constexpr int pitch(int slots) {
     int p = L;
-    while (p % slots != W % slots) p++;
+    while (slots % W == 0 ? p % (2 * W) != W : p % slots != W % slots) p++;
     return p;
   }
-  static constexpr bool SPLIT = sizeof(cx<R>) * L * NZ > 36 * 1024;
+  // halves above 36 KB, so that at least four workgroups share a CU: FP64 96^3
+  // x 8 vectors (28-element rows) 57 us with two workgroups, 50 now; halving
+  // further sizes costs the extra barriers' time (128^3 x 8 FP32 54 -> 55.5)
+  static constexpr bool SPLIT =
+      sizeof(cx<R>) * NZ * pitch((int)(256 / sizeof(cx<R>))) > 36 * 1024;
   static constexpr size_t ES = SPLIT ? sizeof(R) : sizeof(cx<R>);
   static constexpr int P = pitch((int)(256 / ES));
   static constexpr size_t BUF = (ES * (size_t)NZ * P + 15) / 16 * 16;

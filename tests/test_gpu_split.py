@@ -12,7 +12,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 GRIDS = [(16, 16, 16), (16, 80, 36), (128, 16, 24), (24, 128, 16), (36, 36, 36), (48, 64, 80),
-         (80, 24, 160), (160, 36, 32), (64, 160, 16), (32, 96, 48), (96, 48, 128)]
+         (80, 24, 160), (160, 36, 32), (64, 160, 16), (32, 96, 48), (96, 48, 128),
+         (16, 96, 96), (24, 160, 80), (16, 160, 160)]
 
 
 @pytest.mark.parametrize("grid", GRIDS)
