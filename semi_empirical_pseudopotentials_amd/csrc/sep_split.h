@@ -512,8 +512,10 @@ struct TileCfg {
   static constexpr size_t BUF = (ES * (size_t)NZ * P + 15) / 16 * 16;
   static constexpr size_t LDS = BUF + sizeof(cx<R>) * LineTw<NZ>::WORDS + sizeof(double) * NZ;
   // waves per SIMD the register budget must allow: 16 and more FP64 points a
-  // thread spill at 4
-  static constexpr int WPE = E * sizeof(cx<R>) > 192 ? 3 : 4;
+  // thread spill at 4; 20 FP32 points run better held to 5 (160^3 x 4: 80 ->
+  // 73 us; six-residue tiles 31.4 -> 32), 16 spill there (128^3 x 8: 53 -> 67)
+  static constexpr int WPE =
+      E * sizeof(cx<R>) > 192 ? 3 : sizeof(R) == 4 && E > 16 && W == 4 ? 5 : 4;
 };
 
 // pden > 0: the factor is kscale / (kin + pden) instead of kin * kscale.
