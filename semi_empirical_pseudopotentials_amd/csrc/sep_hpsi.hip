@@ -1145,6 +1145,13 @@ static bool use_plane(const GridDev &gd, int prec) {
 static bool use_split(const GridDev &gd, int prec) {
   return !gd.force_lines[prec] && gd.fused_form[prec] == SEP_FUSED_PLANE;
 }
+// Whether one application is one kernel (the filter's fused steps run the
+// two-kernel form: their first kernel also starts the next step).
+template <typename R>
+static bool use_box(const GridDev &gd) {
+  return use_split(gd, sizeof(R) == 8 ? SEP_PREC_FP64 : SEP_PREC_FP32) &&
+         box_supported<R>(gd.nx, gd.ny, gd.nz);
+}
 template <typename R>
 static const cx<R> *twid(const GridDev &gd, int axis) {
   return reinterpret_cast<const cx<R> *>(sizeof(R) == 8 ? gd.tw64[axis] : gd.tw32[axis]);
@@ -1180,6 +1187,18 @@ int hpsi_apply(const GridDev &gd, const VecView<R> &in, const VecView<R> &out, c
   Epi<R> epi{pot, alpha, beta, part};
   bool ok = true;
   if (ev) hipEventRecord(ev[0], st);
+  if (use_box<R>(gd)) {
+    // the whole kernel counts as the spectral passes
+    if (ev) hipEventRecord(ev[1], st);
+    ok = box_apply<R>(gd, in, out, epi, nvec, st);
+    if (nblk) *nblk = nvec;
+    if (ev) {
+      hipEventRecord(ev[2], st);
+      hipEventRecord(ev[3], st);
+    }
+    if (!ok) return SEP_ERR_UNSUPPORTED;
+    return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
+  }
   if (use_split(gd, prec)) {
     ok = SplitOps<R>::rows_fwd(nx, ny, nz, in, tb, nvec, twx, st);
   } else if (use_plane(gd, prec)) {
@@ -1303,6 +1322,8 @@ int hpsi_prepare(const GridDev &gd) {
   const int prec = sizeof(R) == 8 ? SEP_PREC_FP64 : SEP_PREC_FP32;
   if (use_split(gd, prec)) {
     if (!spectral<R>(gd, nullptr, 0, nullptr)) return SEP_ERR_UNSUPPORTED;
+    const VecView<R> none{nullptr, nullptr, nullptr, 0};
+    if (use_box<R>(gd)) box_apply<R>(gd, none, none, Epi<R>{}, 0, nullptr);
   } else if (use_plane(gd, prec)) {
     if constexpr (sizeof(R) == 4) {
       VecView<R> none{nullptr, nullptr, nullptr, 0};

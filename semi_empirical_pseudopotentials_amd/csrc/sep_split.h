@@ -786,6 +786,19 @@ bool SplitOps<R>::tile(int nx, int ny, int nz, cx<R> *tb, int nvec, const cx<R> 
   return false;
 }
 
+// Grids whose application runs in one kernel (sep_box.hip): all sides 16, or
+// in FP32 one of them 24.
+template <typename R>
+inline bool box_supported(int nx, int ny, int nz) {
+  const bool sides = (nx == 16 || nx == 24) && (ny == 16 || ny == 24) && (nz == 16 || nz == 24);
+  return sides && (long)nx * ny * nz <= (sizeof(R) == 8 ? 4096 : 6144);
+}
+// That application; the sums of a vector go to part[4 vec].  false: no such
+// form.  nvec == 0: kernel attributes only.
+template <typename R>
+bool box_apply(const GridDev &gd, const VecView<R> &in, const VecView<R> &out, const Epi<R> &epi,
+               int nvec, hipStream_t st);
+
 // compiled in sep_split64.hip and sep_split32.hip
 extern template struct SplitOps<double>;
 extern template struct SplitOps<float>;
