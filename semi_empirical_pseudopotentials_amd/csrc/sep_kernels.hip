@@ -15,14 +15,16 @@ namespace sep {
 // replaces the linear segment by the cubic Hermite interpolant of
 // cubic_weights() (same segment, same cutoff), a C^1 function of |r - R|.
 //
-// One workgroup per brick of 16 x 4 x 4 points.  Each 256 atoms are tested
+// One workgroup per brick of 8 x 8 x 4 points, a cube of 4 per wave.  Each 256 atoms are tested
 // against the brick (distance to its box against the table's range) and the
 // survivors gathered in LDS in file order, so a point meets the atoms near
 // its brick only; the skipped ones add nothing in the reference either, so
 // the sum is the same bit for bit.  Bound by the FP64 divisions and square
 // roots of the pairs in range: 1667 atoms on 128^3 (CdSe, 4 nm) 5.73 ms with
-// every atom at every point, 0.32 ms now.
-constexpr int VB_X = 16, VB_Y = 4, VB_Z = 4;
+// every atom at every point, 0.31 ms in bricks of 16 x 4 x 4 with rows of 16 a
+// wave, 0.28 with cubes of 4 (more of an atom's waves are skipped whole), 0.26
+// in the more compact bricks (cubic tables 0.40, 0.35 and 0.34).
+constexpr int VB_X = 8, VB_Y = 8, VB_Z = 4;
 __global__ void __launch_bounds__(256) k_build_potential(
     int nx, int ny, int nz, double xmin, double ymin, double zmin, double dx, double dy, double dz,
     long natom, const double *__restrict__ xyz, const int *__restrict__ type,
@@ -53,7 +55,7 @@ __global__ void __launch_bounds__(256) k_build_potential(
     ax[VB_X + VB_Y + t - 128] = p;
   }
   __syncthreads();
-  const int qx = t % VB_X, qy = t / VB_X % VB_Y, qz = t / (VB_X * VB_Y);
+  const int qx = 4 * (wave % 2) + lane % 4, qy = 4 * (wave / 2) + lane / 4 % 4, qz = lane / 16;
   const double px = ax[qx], py = ax[VB_X + qy], pz = ax[VB_X + VB_Y + qz];
   const double xa = ax[0], xb = ax[VB_X - 1], ya = ax[VB_X], yb = ax[VB_X + VB_Y - 1],
                za = ax[VB_X + VB_Y], zb = ax[VB_X + VB_Y + VB_Z - 1];

@@ -1,4 +1,4 @@
-"""V(r) gathers the atoms near each brick of 16 x 4 x 4 points
+"""V(r) gathers the atoms near each brick of 8 x 8 x 4 points
 (k_build_potential): the sum must stay that of every atom at every point, bit
 for bit with linear tables, on grids that end inside a brick, with atoms
 outside the box, tables of different ranges (one shorter than a grid spacing)
