@@ -14,6 +14,7 @@
 // (measured on gfx950).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "sep_internal.h"
@@ -109,6 +110,7 @@ __global__ void __launch_bounds__(256) k_gram_t(const R *__restrict__ A, long ld
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int li = lane & 15, h = lane >> 4;
   const long i0 = (long)bi * GT + 64 * (w >> 1), j0 = (long)bj * BW + 16 * TJ * (w & 1);
+  if (i0 >= m || j0 >= mb) return;  // the wave's whole quadrant lies outside C
   const long g0 = (long)z * kc;
   const long g1 = g0 + kc < K ? g0 + kc : K;
   // rows outside the operands read row 0 (their products land in C
@@ -197,17 +199,32 @@ __global__ void __launch_bounds__(256) k_gram_t(const R *__restrict__ A, long ld
       }
 }
 
-__global__ void k_sum_chunks(const double *work, long nchunk, long len, double *out) {
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len; e += (long)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (long c = 0; c < nchunk; c++) s += work[c * len + e];
-    out[e] = s;
+// out[e] = sum over the chunks of work[c len + e]: 64 elements per workgroup,
+// eight groups of lanes take an eighth of the chunks each, added in order
+__global__ void __launch_bounds__(512) k_sum_chunks(const double *work, long nchunk, long len,
+                                                    double *out) {
+  __shared__ double part[8][64];
+  const int l = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const long e = (long)blockIdx.x * 64 + l;
+  double s = 0.0;
+  if (e < len) {
+#pragma unroll 8
+    for (long c = nchunk * q / 8; c < nchunk * (q + 1) / 8; c++) s += work[c * len + e];
   }
+  part[q][l] = s;
+  __syncthreads();
+  if (q > 0 || e >= len) return;
+  for (int k = 1; k < 8; k++) s += part[k][l];
+  out[e] = s;
 }
 
 // Shape of one Gram launch.  Block tile GT x bw; chunk count a multiple of 8
-// (one group per XCD) giving >= ~2048 blocks, chunks of at least 4096
-// contraction indices.
+// (one group per XCD) giving >= ~2048 blocks.  A chunk has at least 4096
+// contraction indices, or fewer for few states, whose single tile would leave
+// most CUs idle: so many that a chunk reads 16 times the bytes of its partial
+// sums, and 64 MB of partial sums in all.  64 states of 48^3 in FP64 with 32
+// workgroups 433 us, with 216 70 us; the whole call in FP32 at 64 states of
+// 128^3 776 -> 383 us (at 256 states the chunks are as before).
 struct GramShape {
   int tj, ntiles, nch;
   long kc;
@@ -219,7 +236,8 @@ static GramShape gram_shape(long m, long mb, long K, bool sym, int bw) {
   g.tj = (int)((mb + bw - 1) / bw);
   g.ntiles = sym ? ti * (ti + 1) / 2 : ti * g.tj;
   long want = (2048 + g.ntiles - 1) / g.ntiles;
-  long maxch = (K + 4095) / 4096;
+  const long kmin = std::max(512L, 16 * m * mb / (m + mb));
+  long maxch = std::max((K + 4095) / 4096, std::min((K + kmin - 1) / kmin, (8L << 20) / (m * mb)));
   if (want > maxch) want = maxch;
   if (want < 1) want = 1;
   want = (want + 7) / 8 * 8;
@@ -275,9 +293,8 @@ int gram_launch(const R *A, long lda, long m, const R *B, long ldb, long mb, lon
     hipLaunchKernelGGL((k_gram_t<R, false, TJ, ST>), dim3(nblk), dim3(256), 0, st, A, lda, m, B,
                        ldb, mb, K, g.kc, g.tj, g.ntiles, g.nch, sym ? 1 : 0, work);
   const long len = m * mb;
-  unsigned nb = (unsigned)((len + 255) / 256);
-  if (nb > 4096) nb = 4096;
-  hipLaunchKernelGGL(k_sum_chunks, dim3(nb), dim3(256), 0, st, work, (long)g.nch, len, C_d);
+  hipLaunchKernelGGL(k_sum_chunks, dim3((unsigned)((len + 63) / 64)), dim3(512), 0, st, work,
+                     (long)g.nch, len, C_d);
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
@@ -799,6 +816,7 @@ __global__ void k_sum_chunks_dd(const double *whi, const double *wlo, long nchun
 #pragma clang fp contract(off)
   for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < len; e += (long)gridDim.x * blockDim.x) {
     double hi = 0.0, lo = 0.0;
+#pragma unroll 8
     for (long c = 0; c < nchunk; c++) {
       double x = whi[c * len + e];
       double s = hi + x, bb = s - hi;
@@ -813,21 +831,24 @@ __global__ void k_sum_chunks_dd(const double *whi, const double *wlo, long nchun
   }
 }
 
-// contraction chunk of the double-double Gram: >= 8 chunks where N allows
-static long dd_chunk(long N) {
+// contraction chunk of the double-double Gram: >= 8 chunks where N allows, and
+// ~1024 workgroups for few states (64 of 48^3: 140 workgroups 530 us, 1080 203 us)
+static long dd_chunk(long m, long N) {
+  const long t = (m + 15) / 16, tiles = t * (t + 1) / 2;
   long kc = 65536;
   while (kc > 4096 && (N + kc - 1) / kc < 8) kc /= 2;
+  while (kc > 1024 && tiles * ((N + kc - 1) / kc) < 1024) kc /= 2;
   return kc;
 }
 
 long gram_dd_work_len(long m, long N) {
-  const long kc = dd_chunk(N);
+  const long kc = dd_chunk(m, N);
   return 2 * ((N + kc - 1) / kc) * m * m;
 }
 
 int gram_dd_dev(const double *A, long m, long N, double *hi_d, double *lo_d, double *work,
                 long work_len, hipStream_t st) {
-  long kc = dd_chunk(N);
+  long kc = dd_chunk(m, N);
   long nch = (N + kc - 1) / kc;
   if (2 * nch * m * m > work_len) return SEP_ERR_NOMEM;
   double *whi = work, *wlo = work + nch * m * m;
