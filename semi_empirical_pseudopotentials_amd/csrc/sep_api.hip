@@ -813,6 +813,26 @@ static int zero_dev(void *p, size_t bytes, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
+// Newton vectors of one ring block of per_k bytes a vector: up to 1024 in 32
+// GB, beyond that what the targets need.  The accumulators' read and write of
+// 16 ms bytes a point comes once per block: 12 vectors a target keep it at 1.3
+// bytes a step, beside the 26 (FP32) that a step moves.  A deeper ring gains
+// nothing (128^3, ms a filter at 256 / 384 / 1024 vectors: 16 states x 32
+// targets FP32 653 / 633 / 650, one target FP64 84.7 / 86.4 / 84.6; below 256
+// launches get short: 128 vectors 87.3) and its memory costs more than the
+// filter where it is not at hand: the first filter of 512 steps after other
+// contexts have come and gone 1.9-2.3 s with 69 GB, 0.09-0.6 s with 34.  The test
+// hook SEP_RING_DEPTH lowers the bound, so that short filters span several
+// blocks.
+static long ring_depth(long nc, long ms, double per_k) {
+  const long need = std::max(256L, (12 * ms + 127) / 128 * 128);
+  const long fit = (long)((double)(1L << 35) / per_k) / 64 * 64;
+  long k = std::min(1024L, std::max(need, fit));
+  const char *env = getenv("SEP_RING_DEPTH");
+  if (env && atol(env) >= 1) k = std::min(k, atol(env));
+  return std::min(nc, k);
+}
+
 template <typename R>
 static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool psi0_on_device,
                         long ns, const double *an, const double *zn, long nc, long ms, double vmin,
@@ -828,21 +848,15 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   f.dE_1 = 4.0 / dE;
   f.nvec = (ns + 1) / 2;
   const long S2 = 2 * f.nvec;
-  // K Newton vectors are accumulated per pass over the ring; the
-  // accumulators move 2 ms 8 / K bytes per real-state point per step.  The
-  // ring holds up to 1024 vectors in up to 160 GB and 60 % of the free
-  // device memory (the ring already held by this context counts as free):
-  // at 128^3 with 16 states, 1024 complex64 vectors (137 GB) filter 4 %
-  // faster than 512.  The test hook SEP_RING_DEPTH lowers the bound on K, so
-  // that short filters span several ring blocks.
+  // K Newton vectors are accumulated per pass over the ring (ring_depth), which
+  // takes up to 160 GB and 60 % of the free device memory (the ring already
+  // held by this context counts as free).
   // ring_cap > 0: the bound a batch of grids planned for this one
   size_t mfree = 0, mtotal = 0;
   if (ring_cap <= 0.0 && hipMemGetInfo(&mfree, &mtotal) != hipSuccess) mfree = 0;
   const double cap =
       ring_cap > 0.0 ? ring_cap : std::min(160.0e9, 0.6 * ((double)mfree + (double)c->ring_bytes));
-  const char *kenv = getenv("SEP_RING_DEPTH");
-  const long kmax = kenv && atol(kenv) >= 1 && atol(kenv) <= 1024 ? atol(kenv) : 1024;
-  long K = nc < kmax ? nc : kmax;
+  long K = ring_depth(nc, ms, (double)S2 * N * sizeof(R));
   while (K > 8 && (double)K * S2 * N * sizeof(R) > cap) K /= 2;
   // ring layout [state][Newton vector][point]: row (s, k) at s * K * N + k * N,
   // so the accumulation walks each state's K rows within K * N elements;
@@ -1118,15 +1132,13 @@ static int filter_batch_impl(int nd, sep_ctx *const *ctxs, const void *const *ps
     size_t mfree = 0, mtotal = 0;
     if (hipMemGetInfo(&mfree, &mtotal) == hipSuccess) avail = (double)mfree;
   }
-  long kmax = 0;
+  long K = 0;
   for (int d = 0; d < nd; d++) {
     per_k[d] = (double)(2 * ((ns[d] + 1) / 2)) * (double)ctxs[d]->gd.N * sizeof(R);
     sum_k += per_k[d];
     avail += (double)ctxs[d]->ring_bytes;
-    kmax = std::max(kmax, nc[d]);
+    K = std::max(K, ring_depth(nc[d], ms[d], per_k[d]));
   }
-  const char *kenv = getenv("SEP_RING_DEPTH");
-  long K = std::min(kmax, (kenv && atol(kenv) >= 1 && atol(kenv) <= 1024) ? atol(kenv) : 1024L);
   const double total = std::min(160.0e9 * nd, 0.6 * avail);
   while (K > 8 && (double)K * sum_k > total) K /= 2;
   for (int d = 0; d < nd; d++) {
