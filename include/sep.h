@@ -196,12 +196,14 @@ int sep_filter_batch(int ndots, sep_ctx *const *ctxs, const void *const *psi0_de
 /* ------------------------------------------------------------ measurement */
 /* Times the H.psi passes on nvec resident complex vectors (random data) with
  * HIP events on the context's stream: kernel_ms[0..3] = average duration of
- * pass A (xy forward), pass B (z pencils with k^2), pass C (xy backward +
+ * pass A (forward rows, or xy forward), pass B (tiles or z pencils with k^2), pass C (backward +
  * Newton epilogue) and one accumulation launch (K = 64 Newton vectors,
  * ms targets, 2 nvec real states); kernel_ms[4] = passes A+B+C timed as one
  * span; kernel_ms[5] = one Newton step of the filter loop's split form
  * (the spectral passes and the kernel that fuses pass C with the next step's
- * pass A), 0 where the grid has no split form.  kernel_ms holds 6 values.  No counterpart in the reference (it only prints clock() totals,
+ * pass A), 0 where the grid has no split form.  Where one kernel runs the
+ * whole application (16^3, FP32 with one side 24), pass B is that kernel.
+ * kernel_ms holds 6 values.  No counterpart in the reference (it only prints clock() totals,
  * filter/main.c:63-66,91-100). */
 int sep_bench_hpsi(sep_ctx *ctx, int precision, long nvec, long ms, long iters,
                    double *kernel_ms);
@@ -213,14 +215,14 @@ int sep_bench_hpsi(sep_ctx *ctx, int precision, long nvec, long ms, long iters,
 int sep_bench_copy(sep_ctx *ctx, long nbytes, long iters, double *gbs);
 
 /* Live kernel timing of the filter loop.  While on, sep_filter/sep_filter_dev
- * record HIP events on the context's stream around the three H.psi passes of
+ * record HIP events on the context's stream around the H.psi kernels of
  * one Newton step per ring block, and around that block's accumulation
  * launch (one host wait per block).  sep_set_timing resets the sums;
  * sep_get_timing returns avg_ms[0..3] = passes A, B, C and the accumulation
  * of a full ring block (where the loop runs pass C fused with the next
  * step's pass A, avg_ms[0] = 0, avg_ms[1] covers the spectral passes -- the
- * row + line family's y lines, z pencils and y lines -- and avg_ms[2] the
- * fused kernel), and
+ * two-kernel form's tiles, the row + line family's y lines, z pencils and y
+ * lines -- and avg_ms[2] the fused kernel), and
  * samples[0..1] = the number of sampled steps and
  * of sampled full blocks.  No counterpart in the reference (it only prints
  * clock() totals, filter/main.c:63-66,91-100). */
@@ -244,8 +246,8 @@ int sep_trim(sep_ctx *ctx);
  * counterpart in the reference's function interface. */
 int sep_set_filter_lanes(sep_ctx *ctx, int lanes);
 /* Autotuner: times the H.psi passes of this grid in `precision` on nvec
- * resident random vectors with the plane kernels (when the line length has
- * them) and with the row + strided-line kernels, and keeps the faster family
+ * resident random vectors with the default two-kernel form and, on grids with a
+ * plane family, with the row + strided-line kernels, and keeps the faster family
  * for this context and precision.  ms_plane (-1 when unavailable) and
  * ms_lines (optional) get the measured time of one Newton step's H.psi in
  * the filter loop's split form (A + B + C where a family has none).
@@ -254,13 +256,13 @@ int sep_set_filter_lanes(sep_ctx *ctx, int lanes);
  * context's state and ring buffers as scratch: call it before filtering. */
 int sep_autotune(sep_ctx *ctx, int precision, long nvec, double *ms_plane, double *ms_lines);
 /* H.psi kernel families of sep_set_hpsi_family. */
-#define SEP_HPSI_PLANE 0         /* whole-plane kernels (passes A and C, C fused with A) */
-#define SEP_HPSI_PLANE_CHUNKED 1 /* same, the fused kernel transposing through half a \
+#define SEP_HPSI_PLANE 0         /* the default: two kernels a step, the y lines split \
+                                    between them */
+#define SEP_HPSI_PLANE_CHUNKED 1 /* xy planes in registers, transposed through half a \
                                     plane of LDS so that two workgroups share a CU */
-#define SEP_HPSI_LINES 2         /* row + strided-line kernels */
-#define SEP_HPSI_PLANE_SWIZZLED 3 /* whole-plane kernels, the fused kernel on the \
-                                     xor-swizzled LDS placement that SEP_HPSI_PLANE \
-                                     replaces at complex64 128 x 128 */
+#define SEP_HPSI_LINES 2         /* row + strided-line kernels; on grids without a \
+                                    plane family the default form */
+#define SEP_HPSI_PLANE_SWIZZLED 3 /* whole xy planes in LDS on an xor-swizzled placement */
 #define SEP_HPSI_NFAMILY 4
 /* Selects the H.psi kernel family of this context in `precision`.
  * SEP_ERR_UNSUPPORTED if the grid has no such form (plane families need

@@ -815,17 +815,16 @@ static int zero_dev(void *p, size_t bytes, hipStream_t st) {
 
 // Newton vectors of one ring block of per_k bytes a vector: up to 1024 in 32
 // GB, beyond that what the targets need.  The accumulators' read and write of
-// 16 ms bytes a point comes once per block: 12 vectors a target keep it at 1.3
-// bytes a step, beside the 26 (FP32) that a step moves.  A deeper ring gains
-// nothing (128^3, ms a filter at 256 / 384 / 1024 vectors: 16 states x 32
-// targets FP32 653 / 633 / 650, one target FP64 84.7 / 86.4 / 84.6; below 256
-// launches get short: 128 vectors 87.3) and its memory costs more than the
-// filter where it is not at hand: the first filter of 512 steps after other
-// contexts have come and gone 1.9-2.3 s with 69 GB, 0.09-0.6 s with 34.  The test
-// hook SEP_RING_DEPTH lowers the bound, so that short filters span several
-// blocks.
+// 16 ms bytes a point comes once per block: 32 vectors a target keep it at half
+// a byte a step, beside the 26 (FP32) that a step moves (128^3, 16 states x 32
+// targets x 4096 FP32: 742 ms at 384 vectors, 717 at 1024).  For few targets a
+// deeper ring gains nothing (8 states x 1 target x 512 FP64 at 128 / 256 / 512
+// vectors: 87.3 / 84.7 / 84.6 ms), and its memory costs more than the filter
+// where it is not at hand: the first filter of that case after other contexts
+// have come and gone 1.9-2.3 s with 69 GB, 0.09-0.6 s with 34.  The test hook
+// SEP_RING_DEPTH lowers the bound, so that short filters span several blocks.
 static long ring_depth(long nc, long ms, double per_k) {
-  const long need = std::max(256L, (12 * ms + 127) / 128 * 128);
+  const long need = std::max(256L, 32 * ms);
   const long fit = (long)((double)(1L << 35) / per_k) / 64 * 64;
   long k = std::min(1024L, std::max(need, fit));
   const char *env = getenv("SEP_RING_DEPTH");
