@@ -35,7 +35,7 @@ struct Epi {
   const R *pot;   // V on the grid
   double alpha, beta;
   double *part;   // per-block partial sums (4 per block) or nullptr
-  // spinor filter (FP64 whole-plane fused kernel only): psi_j += so_alpha *
+  // spinor filter (FP64 backward rows that start the next step): psi_j += so_alpha *
   // (V_so psi_{j-1}) at the grid points in a spin-orbit list, so_map[g] the
   // point's row of so_g (4 doubles per spinor: up re, im, dn re, im) or -1
   const int *so_map = nullptr;
