@@ -671,9 +671,12 @@ int sep_energy_range_log(sep_ctx *c, double vmin, double *dE, double *emax, long
   // norms follow from the sums <w_k|w_(k+1)> and |w_(k+1)|^2, so that ER_BATCH
   // applications are queued before the host waits for their sums (per
   // iteration it otherwise waited, sent the norm back and ran a copy and a
-  // scaling pass: 64^3 55 us an iteration, 24 us now).  alpha follows the
-  // last batch's growth, which keeps |w| near 1; the applications past the
-  // converged one (at most ER_BATCH - 1) are not used.
+  // scaling pass: 64^3 55 us an iteration, 24 us now).  The first application
+  // is looked at alone; the next ones' alpha is the inverse of the last growth
+  // seen, and at the start of a batch the norm that has gathered is taken out,
+  // so that |w| stays within the growth's change over one batch, whatever the
+  // units and the depth of V.  alpha is a power of two and rounds nothing.  The
+  // applications past the converged one (at most ER_BATCH - 1) are not used.
   constexpr int ER_BATCH = 8;
   const size_t slot = ((size_t)c->gd.ny * c->gd.nz + c->gd.nz) * 4;  // as apply_views
   RCHK(ensure_states(c, 2, 2));
@@ -682,26 +685,31 @@ int sep_energy_range_log(sep_ctx *c, double vmin, double *dE, double *emax, long
   double *w = c->states2, *hw = w + N;
   HIPCHK(c, hipMemcpyAsync(w, re.data(), sizeof(double) * N, hipMemcpyHostToDevice, c->st));
   double ene = 0.0 + 0.1, ene_old = 0.0;
-  double alpha = 1.0, n2 = 1.0 / c->dv;  // |w|^2 (the start vector is normalised)
-  double hn = 0.0;                       // |H psi|^2 of the iterate the next energy belongs to
-  long i = -1;                           // application -1 only gives the first iterate's norm
+  double rate = 1.0, n2 = 1.0 / c->dv;  // n2 = |w|^2 (the start vector is normalised)
+  double hn = 0.0;                      // |H psi|^2 of the iterate the next energy belongs to
+  long i = -1;                          // application -1 only gives the first iterate's norm
   int rc = SEP_OK;
   std::vector<double> h;
   bool more = true;
   while (rc == SEP_OK && more) {
     long nblk = 0;
-    for (int b = 0; b < ER_BATCH && rc == SEP_OK; b++) {
+    const double w2 = n2 * c->dv;
+    const double first = w2 > 0.0 && std::isfinite(w2) ? ldexp(rate, -ilogb(w2) / 2) : rate;
+    const int nb = i < 0 ? 1 : ER_BATCH;
+    for (int b = 0; b < nb && rc == SEP_OK; b++) {
       VecView<double> in{w, nullptr, nullptr, N}, out{hw, nullptr, nullptr, N};
       rc = hpsi_apply<double>(c->gd, in, out, reinterpret_cast<cx<double> *>(c->tb), c->pot64, 1,
-                              alpha, 0.0, c->scr + (size_t)b * nblk * 4, &nblk, c->st);
+                              b == 0 ? first : rate, 0.0, c->scr + (size_t)b * nblk * 4, &nblk,
+                              c->st);
       std::swap(w, hw);
     }
     if (rc != SEP_OK) return fail(c, rc, "energy range: H.psi launch failed");
-    h.resize((size_t)nblk * 4 * ER_BATCH);
+    h.resize((size_t)nblk * 4 * nb);
     HIPCHK(c, hipMemcpyAsync(h.data(), c->scr, sizeof(double) * h.size(), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     double grow = 1.0;
-    for (int b = 0; b < ER_BATCH && more; b++) {
+    for (int b = 0; b < nb && more; b++) {
+      const double alpha = b == 0 ? first : rate;
       double s0 = 0.0, s2 = 0.0;
       for (long k = 0; k < nblk; k++) {
         s0 += h[((size_t)b * nblk + k) * 4];
@@ -717,13 +725,13 @@ int sep_energy_range_log(sep_ctx *c, double vmin, double *dE, double *emax, long
           log[3 * i + 2] = norma;
         }
       }
-      hn = s2 / (alpha * alpha * n2);
+      hn = s2 / n2 / alpha / alpha;
       grow = sqrt(s2 / n2);
       n2 = s2;
       i++;
       more = (fabs((ene - ene_old) / ene) > 1.0e-4) && (i < 500);
     }
-    if (grow > 0.0 && std::isfinite(grow)) alpha /= grow;
+    if (grow > 0.0 && std::isfinite(grow)) rate = ldexp(rate, -ilogb(grow));
   }
   if (rc != SEP_OK) return rc;
   if (dE) *dE = 1.1 * (ene - vmin);
