@@ -16,9 +16,17 @@ extern "C" {
  * Returns 0 or k+1 for a non-positive pivot k. */
 int sep_la_chol_dd(long n, const double *hi, const double *lo, double shift, double *R);
 
-/* memcpy of n bytes by up to 8 threads (large host copies: first touches of
- * a fresh destination dominate and run in parallel). */
-void sep_par_copy(void *dst, const void *src, size_t n);
+/* Up to eight threads (the caller's among them, no more than the CPUs it may
+ * run on) that copy large host blocks together: first touches of a fresh
+ * destination dominate such copies and run in parallel.  One download at a time:
+ * wake, any number of runs, rest; the threads sleep outside of it.  NULL, where
+ * memory is short, is a valid team of the caller alone. */
+typedef struct sep_copy_team sep_copy_team;
+sep_copy_team *sep_copy_team_open(void);
+void sep_copy_team_wake(sep_copy_team *t);
+void sep_copy_team_run(sep_copy_team *t, void *dst, const void *src, size_t n);
+void sep_copy_team_rest(sep_copy_team *t);
+void sep_copy_team_close(sep_copy_team *t);
 
 #ifdef __cplusplus
 }
