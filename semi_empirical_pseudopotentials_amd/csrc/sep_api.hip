@@ -846,23 +846,11 @@ static int zero_dev(void *p, size_t bytes, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
-// Newton vectors of one ring block of per_k bytes a vector: up to 1024 in 32
-// GB, beyond that what the targets need.  The accumulators' read and write of
-// 16 ms bytes a point comes once per block: 32 vectors a target keep it at half
-// a byte a step, beside the 26 (FP32) that a step moves (128^3, 16 states x 32
-// targets x 4096 FP32: 742 ms at 384 vectors, 717 at 1024).  For few targets a
-// deeper ring gains nothing (8 states x 1 target x 512 FP64 at 128 / 256 / 512
-// vectors: 87.3 / 84.7 / 84.6 ms), and its memory costs more than the filter
-// where it is not at hand: the first filter of that case after other contexts
-// have come and gone 1.9-2.3 s with 69 GB, 0.09-0.6 s with 34.  The test hook
-// SEP_RING_DEPTH lowers the bound, so that short filters span several blocks.
-static long ring_depth(long nc, long ms, double per_k) {
-  const long need = std::max(256L, 32 * ms);
-  const long fit = (long)((double)(1L << 35) / per_k) / 64 * 64;
-  long k = std::min(1024L, std::max(need, fit));
+// Ring depth bound (sep_ring_depth); the test hook SEP_RING_DEPTH lowers it, so
+// that short filters span several blocks.
+static long ring_most() {
   const char *env = getenv("SEP_RING_DEPTH");
-  if (env && atol(env) >= 1) k = std::min(k, atol(env));
-  return std::min(nc, k);
+  return env && atol(env) >= 1 ? std::min(1024L, atol(env)) : 1024L;
 }
 
 template <typename R>
@@ -880,7 +868,7 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   f.dE_1 = 4.0 / dE;
   f.nvec = (ns + 1) / 2;
   const long S2 = 2 * f.nvec;
-  // K Newton vectors are accumulated per pass over the ring (ring_depth), which
+  // K Newton vectors are accumulated per pass over the ring (sep_ring_depth), which
   // takes up to 160 GB and 60 % of the free device memory (the ring already
   // held by this context counts as free).
   // ring_cap > 0: the bound a batch of grids planned for this one
@@ -888,8 +876,8 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   if (ring_cap <= 0.0 && hipMemGetInfo(&mfree, &mtotal) != hipSuccess) mfree = 0;
   const double cap =
       ring_cap > 0.0 ? ring_cap : std::min(160.0e9, 0.6 * ((double)mfree + (double)c->ring_bytes));
-  long K = ring_depth(nc, ms, (double)S2 * N * sizeof(R));
-  while (K > 8 && (double)K * S2 * N * sizeof(R) > cap) K /= 2;
+  long K = sep_ring_depth(nc, ms, (double)S2 * N * sizeof(R), ring_most());
+  while (K > 8 && (double)K * S2 * N * sizeof(R) > cap) K = sep_ring_halve(K);
   // ring layout [state][Newton vector][point]: row (s, k) at s * K * N + k * N,
   // so the accumulation walks each state's K rows within K * N elements;
   // where the allocation fails (memory the free-memory figure promised went
@@ -897,7 +885,7 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   int rc_ring = ensure(c, &c->ring, &c->ring_bytes, sizeof(R) * (size_t)K * S2 * N);
   while (rc_ring != SEP_OK && K > 8) {
     (void)hipGetLastError();  // the failed allocation must not be reported by a later launch
-    K /= 2;
+    K = sep_ring_halve(K);
     rc_ring = ensure(c, &c->ring, &c->ring_bytes, sizeof(R) * (size_t)K * S2 * N);
   }
   RCHK(rc_ring);
@@ -1169,10 +1157,10 @@ static int filter_batch_impl(int nd, sep_ctx *const *ctxs, const void *const *ps
     per_k[d] = (double)(2 * ((ns[d] + 1) / 2)) * (double)ctxs[d]->gd.N * sizeof(R);
     sum_k += per_k[d];
     avail += (double)ctxs[d]->ring_bytes;
-    K = std::max(K, ring_depth(nc[d], ms[d], per_k[d]));
+    K = std::max(K, sep_ring_depth(nc[d], ms[d], per_k[d], ring_most()));
   }
   const double total = std::min(160.0e9 * nd, 0.6 * avail);
-  while (K > 8 && (double)K * sum_k > total) K /= 2;
+  while (K > 8 && (double)K * sum_k > total) K = sep_ring_halve(K);
   for (int d = 0; d < nd; d++) {
     sep_ctx *c = ctxs[d];
     if (c->ring && (double)c->ring_bytes > (double)K * per_k[d]) {

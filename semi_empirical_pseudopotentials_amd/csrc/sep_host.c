@@ -151,6 +151,32 @@ void sep_copy_team_close(sep_copy_team *t) {
   free(t);
 }
 
+/* ========================================================= ring depth */
+/* Up to 1024 vectors in 32 GB, beyond that what the targets need.  The
+ * accumulators' read and write of 16 ms bytes a point comes once per block: 32
+ * vectors a target keep it at half a byte a step, beside the 26 (FP32) that a
+ * step moves (128^3, 16 states x 32 targets x 4096 FP32: 742 ms at 384 vectors,
+ * 717 at 1024).  For few targets a deeper ring gains nothing (8 states x 1
+ * target x 512 FP64 at 128 / 256 / 512 vectors: 87.3 / 84.7 / 84.6 ms), and its
+ * memory costs more than the filter where it is not at hand: the first filter of
+ * that case after other contexts have come and gone 1.9-2.3 s with 69 GB,
+ * 0.09-0.6 s with 34. */
+long sep_ring_depth(long nc, long ms, double per_k, long most) {
+  const long need = 32 * ms > 256 ? 32 * ms : 256;
+  const long fit = (long)((double)(1L << 35) / per_k) / 64 * 64;
+  long k = need > fit ? need : fit;
+  if (k > 1024) k = 1024;
+  if (k > most) k = most;
+  return k < nc ? k : nc;
+}
+
+/* The accumulation's packed kernel takes blocks that start at multiples of 16:
+ * 288 (nine targets) halved to 144, 72, 36 would leave it at the second step. */
+long sep_ring_halve(long k) {
+  const long h = k / 2;
+  return h < 16 ? h : h / 16 * 16;
+}
+
 /* ===================================================== random numbers */
 /* L'Ecuyer two-generator combination with a 32-entry Bays-Durham shuffle;
  * constants as filter/rand.c:11-24. */

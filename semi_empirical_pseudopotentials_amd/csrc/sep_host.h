@@ -16,6 +16,12 @@ extern "C" {
  * Returns 0 or k+1 for a non-positive pivot k. */
 int sep_la_chol_dd(long n, const double *hi, const double *lo, double shift, double *R);
 
+/* Newton vectors of one block of the filter's ring, for nc Newton vectors in
+ * all, ms targets and per_k bytes a vector; at most `most`. */
+long sep_ring_depth(long nc, long ms, double per_k, long most);
+/* The next depth where the memory is short: half of k, in whole sixteens. */
+long sep_ring_halve(long k);
+
 /* Up to eight threads (the caller's among them, no more than the CPUs it may
  * run on) that copy large host blocks together: first touches of a fresh
  * destination dominate such copies and run in parallel.  One download at a time:
