@@ -846,7 +846,7 @@ static int zero_dev(void *p, size_t bytes, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
-// Ring depth bound (sep_ring_depth); the test hook SEP_RING_DEPTH lowers it, so
+// Ring depth bound (sep_ring_plan); the test hook SEP_RING_DEPTH lowers it, so
 // that short filters span several blocks.
 static long ring_most() {
   const char *env = getenv("SEP_RING_DEPTH");
@@ -856,7 +856,7 @@ static long ring_most() {
 template <typename R>
 static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool psi0_on_device,
                         long ns, const double *an, const double *zn, long nc, long ms, double vmin,
-                        double dE, bool so = false, double ring_cap = 0.0) {
+                        double dE, bool so = false, long ring_k = 0) {
   const long N = c->gd.N;
   if (!c->has_pot) return fail(c, SEP_ERR_ARG, "potential not set");
   f.c = c;
@@ -868,16 +868,18 @@ static int filter_start(FilterRun<R> &f, sep_ctx *c, const double *psi0, bool ps
   f.dE_1 = 4.0 / dE;
   f.nvec = (ns + 1) / 2;
   const long S2 = 2 * f.nvec;
-  // K Newton vectors are accumulated per pass over the ring (sep_ring_depth), which
+  // K Newton vectors are accumulated per pass over the ring (sep_ring_plan), which
   // takes up to 160 GB and 60 % of the free device memory (the ring already
   // held by this context counts as free).
-  // ring_cap > 0: the bound a batch of grids planned for this one
-  size_t mfree = 0, mtotal = 0;
-  if (ring_cap <= 0.0 && hipMemGetInfo(&mfree, &mtotal) != hipSuccess) mfree = 0;
-  const double cap =
-      ring_cap > 0.0 ? ring_cap : std::min(160.0e9, 0.6 * ((double)mfree + (double)c->ring_bytes));
-  long K = sep_ring_depth(nc, ms, (double)S2 * N * sizeof(R), ring_most());
-  while (K > 8 && (double)K * S2 * N * sizeof(R) > cap) K = sep_ring_halve(K);
+  // ring_k > 0: the depth that a batch of grids planned for this one
+  long K = ring_k;
+  if (K <= 0) {
+    size_t mfree = 0, mtotal = 0;
+    if (hipMemGetInfo(&mfree, &mtotal) != hipSuccess) mfree = 0;
+    const double per_k = (double)S2 * N * sizeof(R);
+    sep_ring_plan(1, &nc, &ms, &per_k, ring_most(),
+                  std::min(160.0e9, 0.6 * ((double)mfree + (double)c->ring_bytes)), &K);
+  }
   // ring layout [state][Newton vector][point]: row (s, k) at s * K * N + k * N,
   // so the accumulation walks each state's K rows within K * N elements;
   // where the allocation fails (memory the free-memory figure promised went
@@ -1141,29 +1143,25 @@ static int filter_batch_impl(int nd, sep_ctx *const *ctxs, const void *const *ps
   std::vector<hipGraphExec_t> execs(nd, nullptr);
   std::vector<hipGraph_t> graphs(nd, nullptr);
   int rc = SEP_OK;
-  // One ring depth K for all grids: the rings share 60 % of the free memory
-  // (the rings these contexts hold count as free) in proportion to their
-  // bytes per Newton vector, instead of each taking 60 % of what the grids
+  // The rings share 60 % of the free memory (the rings these contexts hold count
+  // as free), planned together instead of each taking 60 % of what the grids
   // before it left.  Rings larger than planned are released first, so the
   // planned ones fit.
   std::vector<double> per_k(nd);
-  double avail = 0.0, sum_k = 0.0;
+  std::vector<long> K(nd);
+  double avail = 0.0;
   {
     size_t mfree = 0, mtotal = 0;
     if (hipMemGetInfo(&mfree, &mtotal) == hipSuccess) avail = (double)mfree;
   }
-  long K = 0;
   for (int d = 0; d < nd; d++) {
     per_k[d] = (double)(2 * ((ns[d] + 1) / 2)) * (double)ctxs[d]->gd.N * sizeof(R);
-    sum_k += per_k[d];
     avail += (double)ctxs[d]->ring_bytes;
-    K = std::max(K, sep_ring_depth(nc[d], ms[d], per_k[d], ring_most()));
   }
-  const double total = std::min(160.0e9 * nd, 0.6 * avail);
-  while (K > 8 && (double)K * sum_k > total) K = sep_ring_halve(K);
+  sep_ring_plan(nd, nc, ms, per_k.data(), ring_most(), std::min(160.0e9 * nd, 0.6 * avail), K.data());
   for (int d = 0; d < nd; d++) {
     sep_ctx *c = ctxs[d];
-    if (c->ring && (double)c->ring_bytes > (double)K * per_k[d]) {
+    if (c->ring && (double)c->ring_bytes > (double)K[d] * per_k[d]) {
       hipStreamSynchronize(c->st);
       hipFree(c->ring);
       c->ring = nullptr;
@@ -1172,8 +1170,7 @@ static int filter_batch_impl(int nd, sep_ctx *const *ctxs, const void *const *ps
   }
   for (int d = 0; d < nd && rc == SEP_OK; d++) {
     rc = filter_start<R>(runs[d], ctxs[d], static_cast<const double *>(psi0[d]), true, ns[d],
-                         an[d], zn[d], nc[d], ms[d], vmin[d], dE[d], false,
-                         (double)K * per_k[d] * (1.0 + 1e-9));
+                         an[d], zn[d], nc[d], ms[d], vmin[d], dE[d], false, K[d]);
     if (rc == SEP_OK) rc = hpsi_prepare<R>(ctxs[d]->gd);
   }
   if (rc == SEP_OK && mode == SEP_BATCH_GRAPH) {

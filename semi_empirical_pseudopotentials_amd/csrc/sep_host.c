@@ -161,7 +161,7 @@ void sep_copy_team_close(sep_copy_team *t) {
  * memory costs more than the filter where it is not at hand: the first filter of
  * that case after other contexts have come and gone 1.9-2.3 s with 69 GB,
  * 0.09-0.6 s with 34. */
-long sep_ring_depth(long nc, long ms, double per_k, long most) {
+static long ring_depth(long nc, long ms, double per_k, long most) {
   const long need = 32 * ms > 256 ? 32 * ms : 256;
   const long fit = (long)((double)(1L << 35) / per_k) / 64 * 64;
   long k = need > fit ? need : fit;
@@ -175,6 +175,25 @@ long sep_ring_depth(long nc, long ms, double per_k, long most) {
 long sep_ring_halve(long k) {
   const long h = k / 2;
   return h < 16 ? h : h / 16 * 16;
+}
+
+/* Grids that want less than the bound keep what they want (all of them at the
+ * deepest one's depth would be planned for memory that they do not take). */
+void sep_ring_plan(int nd, const long *nc, const long *ms, const double *per_k, long most,
+                   double total, long *K) {
+  long bound = 1;
+  for (int d = 0; d < nd; d++) {
+    K[d] = ring_depth(nc[d], ms[d], per_k[d], most);
+    if (K[d] > bound) bound = K[d];
+  }
+  for (;; bound = sep_ring_halve(bound)) {
+    double sum = 0.0;
+    for (int d = 0; d < nd; d++) {
+      if (K[d] > bound) K[d] = bound;
+      sum += (double)K[d] * per_k[d];
+    }
+    if (bound <= 8 || sum <= total) return;
+  }
 }
 
 /* ===================================================== random numbers */

@@ -16,9 +16,11 @@ extern "C" {
  * Returns 0 or k+1 for a non-positive pivot k. */
 int sep_la_chol_dd(long n, const double *hi, const double *lo, double shift, double *R);
 
-/* Newton vectors of one block of the filter's ring, for nc Newton vectors in
- * all, ms targets and per_k bytes a vector; at most `most`. */
-long sep_ring_depth(long nc, long ms, double per_k, long most);
+/* Ring depths (Newton vectors of one block) of nd filters that run together: nc
+ * Newton vectors in all, ms targets and per_k bytes a vector of each, at most
+ * `most`.  Where the rings exceed `total` bytes, the deepest are halved first. */
+void sep_ring_plan(int nd, const long *nc, const long *ms, const double *per_k, long most,
+                   double total, long *K);
 /* The next depth where the memory is short: half of k, in whole sixteens. */
 long sep_ring_halve(long k);
 
