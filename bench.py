@@ -359,7 +359,8 @@ def batched_uneven(sep, decks, read_deck, np, torch, steps=1):
         ctx.build_potential(d["xyz"], d["type"], d["npot"], d["vr"], d["pot"], d["dr"],
                             expot=d["expot"])
         tune_ms, fam, lanes = ctx.autotune_ex(sep.SEP_PREC_FP32, (ns + 1) // 2)
-        names = ("plane", "plane_chunked", "lines", "plane_swizzled")  # SEP_HPSI_* order
+        # SEP_HPSI_* order
+        names = ("plane", "plane_chunked", "lines", "plane_swizzled", "split")
         tune = {"family": names[fam], "lanes": lanes,
                 "ms_per_step": {f: round(float(t), 4) for f, t in
                                 zip(names, tune_ms) if t > 0}}

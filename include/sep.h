@@ -246,29 +246,31 @@ int sep_trim(sep_ctx *ctx);
  * counterpart in the reference's function interface. */
 int sep_set_filter_lanes(sep_ctx *ctx, int lanes);
 /* Autotuner: times the H.psi passes of this grid in `precision` on nvec
- * resident random vectors with the default two-kernel form and, on grids with a
- * plane family, with the row + strided-line kernels, and keeps the faster family
- * for this context and precision.  ms_plane (-1 when unavailable) and
- * ms_lines (optional) get the measured time of one Newton step's H.psi in
- * the filter loop's split form (A + B + C where a family has none).
+ * resident random vectors in the two-kernel form (or the plane form that was
+ * selected) and with the row + strided-line kernels, and keeps the faster
+ * family for this context and precision.  ms_plane and ms_lines (optional) get the measured time of one
+ * Newton step's H.psi of the two, as the filter loop runs it.
  * No counterpart in the reference (FFTW plans with FFTW_ESTIMATE,
  * filter/filter.c:22-23).  Uses the
  * context's state and ring buffers as scratch: call it before filtering. */
 int sep_autotune(sep_ctx *ctx, int precision, long nvec, double *ms_plane, double *ms_lines);
-/* H.psi kernel families of sep_set_hpsi_family. */
-#define SEP_HPSI_PLANE 0         /* the default: two kernels a step, the y lines split \
-                                    between them */
+/* H.psi kernel families of sep_set_hpsi_family.  A context opens with the
+ * two-kernel form on every grid. */
+#define SEP_HPSI_PLANE 0         /* the two-kernel form, by the name it has on grids with \
+                                    square xy planes of a plane length */
 #define SEP_HPSI_PLANE_CHUNKED 1 /* xy planes in registers, transposed through half a \
                                     plane of LDS so that two workgroups share a CU */
-#define SEP_HPSI_LINES 2         /* row + strided-line kernels; on grids without a \
-                                    plane family the default form */
+#define SEP_HPSI_LINES 2         /* row + strided-line kernels */
 #define SEP_HPSI_PLANE_SWIZZLED 3 /* whole xy planes in LDS on an xor-swizzled placement */
-#define SEP_HPSI_NFAMILY 4
+#define SEP_HPSI_SPLIT 4         /* the two-kernel form (y lines split between the \
+                                    kernels), on every grid */
+#define SEP_HPSI_NFAMILY 5
 /* Selects the H.psi kernel family of this context in `precision`.
- * SEP_ERR_UNSUPPORTED if the grid has no such form (plane families need
+ * SEP_ERR_UNSUPPORTED if the grid has no such form (the plane families need
  * nx == ny and a plane length; the chunked and swizzled forms exist for
  * complex64 128 x 128 planes).  All families give the same H.psi to
- * rounding. */
+ * rounding.  sep_get_hpsi_family returns the family that runs: the two-kernel
+ * form is SEP_HPSI_PLANE where that name is accepted, else SEP_HPSI_SPLIT. */
 int sep_set_hpsi_family(sep_ctx *ctx, int precision, int family);
 int sep_get_hpsi_family(sep_ctx *ctx, int precision, int *family);
 /* Autotuner over every family this grid has and over the number of filter
@@ -276,7 +278,8 @@ int sep_get_hpsi_family(sep_ctx *ctx, int precision, int *family);
  * loop's Newton step (H.psi in split form plus the lane split) on nvec
  * resident random vectors, keeps the fastest family and lane count, and
  * returns the time per family (ms[SEP_HPSI_NFAMILY], -1 where the grid has
- * no such form; may be NULL), the chosen family and lane count.  Uses the
+ * no such form or another name for it, as sep_get_hpsi_family; may be NULL),
+ * the chosen family and lane count.  Uses the
  * context's state and ring buffers as scratch: call it before filtering.
  * No counterpart in the reference (FFTW_ESTIMATE plans, filter/filter.c:22-23). */
 int sep_autotune_ex(sep_ctx *ctx, int precision, long nvec, double *ms, int *family, int *lanes);

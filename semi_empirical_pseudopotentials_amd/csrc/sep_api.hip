@@ -2230,42 +2230,31 @@ extern "C" int sep_bench_hpsi(sep_ctx *c, int precision, long nvec, long ms, lon
 }
 
 // Kernel-family choice per grid and precision: time one Newton step's H.psi
-// in the filter loop's split form (spectral passes + fused kernel; A + B + C
-// where a family has no split form) with the plane kernels and with the row +
-// strided-line kernels on nvec resident random vectors (bench_impl); keep the
-// faster.
+// as the filter loop runs it (spectral passes + fused kernel; A + B + C under
+// the hook SEP_SEPARATE_PASSES) in the two-kernel form (or the plane form that
+// was selected) and with the row + strided-line kernels on nvec resident random
+// vectors (bench_impl); keep the faster.
 extern "C" int sep_autotune(sep_ctx *c, int precision, long nvec, double *ms_plane,
                             double *ms_lines) {
   if (!c || nvec < 1 || (precision != SEP_PREC_FP64 && precision != SEP_PREC_FP32))
     return SEP_ERR_ARG;
   if (!c->has_pot) return fail(c, SEP_ERR_ARG, "potential not set");
   HIPCHK(c, hipSetDevice(c->device));
-  double k[6];
-  double tp = -1.0, tl = -1.0;
   const bool had = c->gd.force_lines[precision];
-  if (plane_supported(c->gd.nx, c->gd.ny, precision)) {
-    c->gd.force_lines[precision] = false;
+  double k[6], t[2];
+  for (int lines = 0; lines < 2; lines++) {
+    c->gd.force_lines[precision] = lines != 0;
     const int rc = precision == SEP_PREC_FP64 ? bench_impl<double>(c, nvec, 1, 5, k)
                                               : bench_impl<float>(c, nvec, 1, 5, k);
     if (rc != SEP_OK) {
       c->gd.force_lines[precision] = had;
       return rc;
     }
-    // the filter loop's split step (spectral passes + fused kernel)
-    tp = k[5] > 0.0 && !c->gd.no_fuse ? k[5] : k[4];
+    t[lines] = k[5] > 0.0 && !c->gd.no_fuse ? k[5] : k[4];
   }
-  // a grid outside the plane family keeps its one form (see sep_set_hpsi_family)
-  c->gd.force_lines[precision] = tp > 0.0 || had;
-  const int rc = precision == SEP_PREC_FP64 ? bench_impl<double>(c, nvec, 1, 5, k)
-                                            : bench_impl<float>(c, nvec, 1, 5, k);
-  if (rc != SEP_OK) {
-    c->gd.force_lines[precision] = had;
-    return rc;
-  }
-  tl = k[5] > 0.0 && !c->gd.no_fuse ? k[5] : k[4];
-  if (tp > 0.0) c->gd.force_lines[precision] = !(tp <= tl);
-  if (ms_plane) *ms_plane = tp;
-  if (ms_lines) *ms_lines = tl;
+  c->gd.force_lines[precision] = t[1] < t[0];
+  if (ms_plane) *ms_plane = t[0];
+  if (ms_lines) *ms_lines = t[1];
   return SEP_OK;
 }
 
@@ -2325,6 +2314,8 @@ extern "C" int sep_autotune_ex(sep_ctx *c, int precision, long nvec, double *ms,
   int bf = -1, bl = 1, rc = SEP_OK;
   for (int f = 0; f < SEP_HPSI_NFAMILY && rc == SEP_OK; f++) {
     t_fam[f] = -1.0;
+    // on plane grids PLANE and SPLIT are one form, timed and reported as PLANE
+    if (f == SEP_HPSI_SPLIT && plane_supported(c->gd.nx, c->gd.ny, precision)) continue;
     if (sep_set_hpsi_family(c, precision, f) != SEP_OK) {
       c->err.clear();  // a family this grid does not have is no error here
       continue;
@@ -2378,11 +2369,8 @@ extern "C" int sep_set_hpsi_family(sep_ctx *c, int precision, int family) {
       return SEP_OK;
     }
     case SEP_HPSI_LINES:
-      // where the grid has no plane family, its default form (the two-kernel
-      // split) stands for this one: the five-pass kernels are slower on every
-      // such grid, and the autotuner would otherwise have to fall back on them
-      c->gd.force_lines[precision] = plane_supported(c->gd.nx, c->gd.ny, precision) ||
-                                     getenv("SEP_FORCE_LINE_KERNELS") != nullptr;
+    case SEP_HPSI_SPLIT:
+      c->gd.force_lines[precision] = family == SEP_HPSI_LINES;
       c->gd.fused_form[precision] = SEP_FUSED_PLANE;
       return SEP_OK;
   }
@@ -2392,13 +2380,12 @@ extern "C" int sep_set_hpsi_family(sep_ctx *c, int precision, int family) {
 extern "C" int sep_get_hpsi_family(sep_ctx *c, int precision, int *family) {
   if (!c || !family || (precision != SEP_PREC_FP64 && precision != SEP_PREC_FP32))
     return SEP_ERR_ARG;
-  const bool plane = !c->gd.force_lines[precision] &&
-                     plane_supported(c->gd.nx, c->gd.ny, precision);
   const int form = c->gd.fused_form[precision];
-  *family = !plane                       ? SEP_HPSI_LINES
-            : form == SEP_FUSED_CHUNKED  ? SEP_HPSI_PLANE_CHUNKED
-            : form == SEP_FUSED_SWIZZLED ? SEP_HPSI_PLANE_SWIZZLED
-                                         : SEP_HPSI_PLANE;
+  *family = c->gd.force_lines[precision]                     ? SEP_HPSI_LINES
+            : form == SEP_FUSED_CHUNKED                      ? SEP_HPSI_PLANE_CHUNKED
+            : form == SEP_FUSED_SWIZZLED                     ? SEP_HPSI_PLANE_SWIZZLED
+            : plane_supported(c->gd.nx, c->gd.ny, precision) ? SEP_HPSI_PLANE
+                                                             : SEP_HPSI_SPLIT;
   return SEP_OK;
 }
 

@@ -1123,7 +1123,8 @@ bool hop_supported(int n) {
   return false;
 }
 
-// Grids of the SEP_HPSI_PLANE family: square xy planes of these lengths.
+// Grids on which the default form goes by the name SEP_HPSI_PLANE (square xy
+// planes of these lengths); elsewhere it is SEP_HPSI_SPLIT only.
 bool plane_supported(int nx, int ny, int prec) {
   if (nx != ny) return false;
   switch (nx) {
