@@ -316,21 +316,9 @@ __global__ void __launch_bounds__(W * FftPlan<NZ>::G) k_pencil(cx<R> *tb, long N
 // row <-> column transpose needs block barriers.  Line positions in LDS are
 // placed by PlaneLds (below) so the strided exchange patterns spread over the
 // banks; FP32 threads keep their twiddles in registers (TwFor).
-// If the plane does not fit LDS, the transpose goes through the buffer in
-// NH chunks of NX/NH columns while the plane stays in registers.
 // The spectrum of a plane is stored column-major, Tbuf[z][kx][ky], so that
 // the column phase writes (and the backward column phase reads) contiguous
 // ky runs.
-template <typename R, int NX>
-constexpr int plane_chunks() {
-  // smallest power of two (dividing NX) whose chunk buffer (plus the
-  // twiddle table) fits the 160 KB of LDS of a gfx950 workgroup
-  int nh = 1;
-  while (nh < NX && NX % (2 * nh) == 0 &&
-         sizeof(cx<R>) * ((size_t)NX * (NX / nh + 1) + NX) > 160 * 1024 - 1024)
-    nh *= 2;
-  return nh;
-}
 
 // LDS placement of one plane in the wave-local plane kernels: row y of the
 // (transposed) plane starts at rowbase(y); during the row FFTs element x of
@@ -368,14 +356,10 @@ __global__ void __launch_bounds__(T) k_plane_fwd_w(VecView<R> in, cx<R> *tb, lon
   using PL = FftPlan<NX>;
   constexpr int G = PL::G, E = PL::E, P = PL::P;
   static_assert(64 % G == 0 && NX % 8 == 0, "lines must not straddle wavefronts");
-  constexpr int NH = plane_chunks<R, NX>(), W = NX / NH;
-  using L = PlaneLds<R, NX, NH>;
+  using L = PlaneLds<R, NX, 1>;
   constexpr int LDc = L::LDc;
-  constexpr int RX = T / G;                  // lines per round
-  constexpr int NR = (NX + RX - 1) / RX;     // row rounds
-  constexpr int NCR = (W + RX - 1) / RX;     // column rounds per chunk
-  constexpr int RS = NX + 1;                 // row-exchange slice pitch (NH > 1)
-  static_assert(NH == 1 || RX * RS <= NX * LDc, "row exchange slices exceed the chunk buffer");
+  constexpr int RX = T / G;               // lines per round
+  constexpr int NR = (NX + RX - 1) / RX;  // row rounds, column rounds
   extern __shared__ char smem_raw[];
   cx<R> *buf = reinterpret_cast<cx<R> *>(smem_raw);  // [NX][LDc], row y at L::rowbase(y)
   cx<R> *tw = buf + NX * LDc;
@@ -401,54 +385,51 @@ __global__ void __launch_bounds__(T) k_plane_fwd_w(VecView<R> in, cx<R> *tb, lon
   __syncthreads();
   TwFor<NX, -1, R> tc;
   tc.init(g, tw);
-  // ---- rows: x FFT; the results stay in registers.  Exchanges use the row's
-  // own buffer row (NH == 1) or slice tl of the chunk buffer.
+  // ---- rows: x FFT, exchanged in the row's own buffer row; the results stay
+  // in registers
 #pragma unroll
   for (int r = 0; r < NR; r++) {
     const int row = r * RX + tl;
     const bool act = row < NX;
-    const int base = (NH == 1 ? L::rowbase(act ? row : 0) : tl * RS);
+    const int base = L::rowbase(act ? row : 0);
     auto at = [&](int i) -> cx<R> & { return buf[base + L::xpos(i)]; };
     run_passes_c<NX, -1, 0, P, WaveSync>(v[r], g, act, tc, at);
   }
-  // ---- columns, chunk by chunk
+  // ---- columns
+  __syncthreads();  // the row exchanges are done
 #pragma unroll
-  for (int c = 0; c < NH; c++) {
-    __syncthreads();  // row exchanges / the previous chunk's columns are done
+  for (int r = 0; r < NR; r++) {
+    const int row = r * RX + tl;
+    if (row < NX) {
 #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      const int row = r * RX + tl;
-      if (row < NX) {
+      for (int b = 0; b < E / rl_; b++)
 #pragma unroll
-        for (int b = 0; b < E / rl_; b++)
-#pragma unroll
-          for (int k = 0; k < rl_; k++) {
-            const int kx = out_idx<NX, -1, P - 1>(g, b, k);
-            if (kx / W == c) buf[L::rowbase(row) + (kx - c * W)] = v[r][b * rl_ + k];
-          }
-      }
+        for (int k = 0; k < rl_; k++)
+          buf[L::rowbase(row) + out_idx<NX, -1, P - 1>(g, b, k)] = v[r][b * rl_ + k];
     }
-    __syncthreads();  // the transpose
+  }
+  __syncthreads();  // the transpose
 #pragma unroll
-    for (int cr = 0; cr < NCR; cr++) {
-      const int cl = cr * RX + tl;
-      const bool act = cl < W;
-      const int cs = act ? cl : 0;
-      cx<R> w[E];
-      auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(i) + cs]; };
-      read_in<NX, -1, 0>(w, g, act, at);
-      run_passes_c<NX, -1, 0, P, WaveSync>(w, g, act, tc, at);
-      if (act) {
-        cx<R> *dst = tb + vec * N + pbase + (long)(c * W + cs) * NX;
+  for (int cr = 0; cr < NR; cr++) {
+    const int cl = cr * RX + tl;
+    const bool act = cl < NX;
+    const int cs = act ? cl : 0;
+    cx<R> w[E];
+    auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(i) + cs]; };
+    read_in<NX, -1, 0>(w, g, act, at);
+    run_passes_c<NX, -1, 0, P, WaveSync>(w, g, act, tc, at);
+    if (act) {
+      cx<R> *dst = tb + vec * N + pbase + (long)cs * NX;
 #pragma unroll
-        for (int b = 0; b < E / rl_; b++)
+      for (int b = 0; b < E / rl_; b++)
 #pragma unroll
-          for (int k = 0; k < rl_; k++) dst[out_idx<NX, -1, P - 1>(g, b, k)] = w[b * rl_ + k];
-      }
+        for (int k = 0; k < rl_; k++) dst[out_idx<NX, -1, P - 1>(g, b, k)] = w[b * rl_ + k];
     }
   }
 }
 
+// At 1024 threads the register budget is 128: twiddles come from LDS, and of
+// the epilogue's operands only V is loaded before the row's FFT.
 template <typename R, int NX, int T>
 __global__ void __launch_bounds__(T) k_plane_bwd_w(const cx<R> *tb, VecView<R> pin,
                                                    VecView<R> out, Epi<R> epi, long N, int nz,
@@ -456,14 +437,10 @@ __global__ void __launch_bounds__(T) k_plane_bwd_w(const cx<R> *tb, VecView<R> p
   using PL = FftPlan<NX>;
   constexpr int G = PL::G, E = PL::E, P = PL::P;
   static_assert(64 % G == 0 && NX % 8 == 0, "lines must not straddle wavefronts");
-  constexpr int NH = plane_chunks<R, NX>(), W = NX / NH;
-  using L = PlaneLds<R, NX, NH>;
+  using L = PlaneLds<R, NX, 1>;
   constexpr int LDc = L::LDc;
   constexpr int RX = T / G;
   constexpr int NR = (NX + RX - 1) / RX;
-  constexpr int NCR = (W + RX - 1) / RX;
-  constexpr int RS = NX + 1;
-  static_assert(NH == 1 || RX * RS <= NX * LDc, "row exchange slices exceed the chunk buffer");
   extern __shared__ char smem_raw[];
   cx<R> *buf = reinterpret_cast<cx<R> *>(smem_raw);
   cx<R> *tw = buf + NX * LDc;
@@ -473,106 +450,64 @@ __global__ void __launch_bounds__(T) k_plane_bwd_w(const cx<R> *tb, VecView<R> p
   const int tl = threadIdx.x / G, g = threadIdx.x % G;
   constexpr int r0 = Pass<NX, 1>::radix(0);
   constexpr int rl_ = Pass<NX, 1>::radix(P - 1);
-  constexpr int NVR = NH == 1 ? 1 : NR;  // row inputs held in registers
-  cx<R> v[NVR][E];
-  // at 1024 threads the register budget is 128: twiddles come from LDS
-  using TwB = typename std::conditional<(T >= 1024), TwTable<NX, 1, R>, TwFor<NX, 1, R>>::type;
-  TwB tc;
+  TwTable<NX, 1, R> tc;
+  // ---- columns: load, y FFT, into the buffer
+  {
+    cx<R> w[NR][E];
 #pragma unroll
-  for (int c = 0; c < NH; c++) {
-    // ---- columns of chunk c: load, y FFT, into the buffer
-    cx<R> w[NCR][E];
-#pragma unroll
-    for (int cr = 0; cr < NCR; cr++) {
+    for (int cr = 0; cr < NR; cr++) {
       const int cl = cr * RX + tl;
-      if (cl < W) {
-        const cx<R> *src = tb + vec * N + pbase + (long)(c * W + cl) * NX;
+      if (cl < NX) {
+        const cx<R> *src = tb + vec * N + pbase + (long)cl * NX;
 #pragma unroll
         for (int b = 0; b < E / r0; b++)
 #pragma unroll
           for (int k = 0; k < r0; k++) w[cr][b * r0 + k] = src[in_idx<NX, 1, 0>(g, b, k)];
       }
     }
-    if (c == 0) {
-      load_tw<R, NX>(tw, twg);
-      __syncthreads();
-      tc.init(g, tw);
-    } else {
-      __syncthreads();  // the previous chunk's gather is done
-    }
+    load_tw<R, NX>(tw, twg);
+    __syncthreads();
+    tc.init(g, tw);
 #pragma unroll
-    for (int cr = 0; cr < NCR; cr++) {
+    for (int cr = 0; cr < NR; cr++) {
       const int cl = cr * RX + tl;
-      const bool act = cl < W;
+      const bool act = cl < NX;
       const int cs = act ? cl : 0;
       auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(i) + cs]; };
       run_passes_c<NX, 1, 0, P, WaveSync>(w[cr], g, act, tc, at);
       WaveSync::sync();
       write_out<NX, 1, P - 1>(w[cr], g, act, at);
     }
-    __syncthreads();  // the transpose
-    if constexpr (NH > 1) {
-      // gather this chunk's x positions of every row this thread owns
-#pragma unroll
-      for (int r = 0; r < NR; r++) {
-        const int row = r * RX + tl;
-        if (row < NX) {
-#pragma unroll
-          for (int b = 0; b < E / r0; b++)
-#pragma unroll
-            for (int k = 0; k < r0; k++) {
-              const int x = in_idx<NX, 1, 0>(g, b, k);
-              if (x / W == c) v[r][b * r0 + k] = buf[L::rowbase(row) + (x - c * W)];
-            }
-        }
-      }
-    }
   }
-  if constexpr (NH > 1) __syncthreads();  // the buffer is free for the row exchanges
+  __syncthreads();  // the transpose
   double s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int r = 0; r < NR; r++) {
     const int row = r * RX + tl;
     const bool act = row < NX;
     const int rs = act ? row : 0;
-    // psi_{j-1} and V of the row are loaded before the FFT (in flight
-    // during it); at 1024 threads (register budget 128) only V is, psi_{j-1}
-    // after the FFT
-    constexpr bool early = T < 1024;
     cx<R> p[E];
     R V[E];
     if (act) {
 #pragma unroll
       for (int b = 0; b < E / rl_; b++)
 #pragma unroll
-        for (int k = 0; k < rl_; k++) {
-          const long gi = pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k);
-          if (early) p[b * rl_ + k] = pin.ld(vec, gi);
-          V[b * rl_ + k] = epi.pot[gi];
-        }
+        for (int k = 0; k < rl_; k++)
+          V[b * rl_ + k] = epi.pot[pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k)];
     }
-    cx<R> *x = v[NH == 1 ? 0 : r];
-    if constexpr (NH == 1) {
-      // the row is in the buffer (at L::rowbase(y), x in natural order); the
-      // exchanges then run in place in that row at the permuted positions
-      auto at0 = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + i]; };
-      read_in<NX, 1, 0>(x, g, act, at0);
-      auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + L::xpos(i)]; };
-      run_passes_c<NX, 1, 0, P, WaveSync>(x, g, act, tc, at);
-    } else {
-      auto at = [&](int i) -> cx<R> & { return buf[tl * RS + lds_swz(i)]; };
-      run_passes_c<NX, 1, 0, P, WaveSync>(x, g, act, tc, at);
-    }
+    // the row is in the buffer (at L::rowbase(y), x in natural order); the
+    // exchanges then run in place in that row at the permuted positions
+    cx<R> x[E];
+    auto at0 = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + i]; };
+    read_in<NX, 1, 0>(x, g, act, at0);
+    auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + L::xpos(i)]; };
+    run_passes_c<NX, 1, 0, P, WaveSync>(x, g, act, tc, at);
     if (act) {
-      if constexpr (!early) {
 #pragma unroll
-        for (int b = 0; b < E / rl_; b++)
+      for (int b = 0; b < E / rl_; b++)
 #pragma unroll
-          for (int k = 0; k < rl_; k++) {
-            const long gi = pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k);
-            p[b * rl_ + k] = pin.ld(vec, gi);
-          }
-      }
+        for (int k = 0; k < rl_; k++)
+          p[b * rl_ + k] = pin.ld(vec, pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k));
 #pragma unroll
       for (int b = 0; b < E / rl_; b++)
 #pragma unroll
@@ -593,8 +528,8 @@ __device__ __forceinline__ int opaque_int(int x) {
   return x;
 }
 
-// Pass C of Newton step j fused with pass A of step j+1 (whole-plane buffer,
-// NH == 1).  The epilogue's psi_j is stored (the ring slot the accumulation
+// Pass C of Newton step j fused with pass A of step j+1 (whole-plane buffer).
+// The epilogue's psi_j is stored (the ring slot the accumulation
 // reads) and, still in registers, transformed forward -- x rows in each row's
 // own buffer row, then y columns -- into plane z of the spectrum buffer,
 // which this block alone read at its start.  Saves pass A's read of psi_j;
@@ -606,7 +541,6 @@ __global__ void __launch_bounds__(T) k_plane_bwd_fwd_w(cx<R> *tb, VecView<R> pin
   using PL = FftPlan<NX>;
   constexpr int G = PL::G, E = PL::E, P = PL::P;
   static_assert(64 % G == 0 && NX % 8 == 0, "lines must not straddle wavefronts");
-  static_assert(plane_chunks<R, NX>() == 1, "the fused kernel holds the whole plane in LDS");
   using L = PlaneLds<R, NX, 1>;
   constexpr int LDc = L::LDc;
   constexpr int RX = T / G;
@@ -622,13 +556,10 @@ __global__ void __launch_bounds__(T) k_plane_bwd_fwd_w(cx<R> *tb, VecView<R> pin
   constexpr int r0b = Pass<NX, 1>::radix(0);
   constexpr int rlb = Pass<NX, 1>::radix(P - 1);
   constexpr int rlf = Pass<NX, -1>::radix(P - 1);
-  // psi_{j-1} before the row FFT only below 1024 threads (at 1024 it fits
-  // the registers but measured 5 % slower: 138 against 132 us at 128^3)
-  constexpr bool early = T < 1024;
-  using TwB = typename std::conditional<(T >= 1024), TwTable<NX, 1, R>, TwFor<NX, 1, R>>::type;
-  using TwF = typename std::conditional<(T >= 1024), TwTable<NX, -1, R>, TwFor<NX, -1, R>>::type;
-  TwB tcb;
-  TwF tcf;
+  // psi_{j-1} is loaded after the row FFT (before it, it fits the registers but
+  // measured 5 % slower: 138 against 132 us at 128^3)
+  TwTable<NX, 1, R> tcb;
+  TwTable<NX, -1, R> tcf;
   // ---- inverse y FFT of the columns (pass C)
   {
     cx<R> w[NR][E];
@@ -675,11 +606,8 @@ __global__ void __launch_bounds__(T) k_plane_bwd_fwd_w(cx<R> *tb, VecView<R> pin
 #pragma unroll
       for (int b = 0; b < E / rlb; b++)
 #pragma unroll
-        for (int k = 0; k < rlb; k++) {
-          const long gi = pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k);
-          if (early) p[b * rlb + k] = pin.ld(vec, gi);
-          V[b * rlb + k] = epi.pot[gi];
-        }
+        for (int k = 0; k < rlb; k++)
+          V[b * rlb + k] = epi.pot[pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k)];
     }
     cx<R> x[E];
     auto at0 = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + i]; };
@@ -687,31 +615,17 @@ __global__ void __launch_bounds__(T) k_plane_bwd_fwd_w(cx<R> *tb, VecView<R> pin
     auto at = [&](int i) -> cx<R> & { return buf[L::rowbase(rs) + L::xpos(i)]; };
     run_passes_c<NX, 1, 0, P, WaveSync>(x, g, act, tcb, at);
     if (act) {
-      if constexpr (!early) {
 #pragma unroll
-        for (int b = 0; b < E / rlb; b++)
+      for (int b = 0; b < E / rlb; b++)
 #pragma unroll
-          for (int k = 0; k < rlb; k++) {
-            const long gi = pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k);
-            p[b * rlb + k] = pin.ld(vec, gi);
-          }
-      }
+        for (int k = 0; k < rlb; k++)
+          p[b * rlb + k] = pin.ld(vec, pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k));
 #pragma unroll
       for (int b = 0; b < E / rlb; b++)
 #pragma unroll
         for (int k = 0; k < rlb; k++) {
           const long gi = pbase + rs * NX + out_idx<NX, 1, P - 1>(g, b, k);
           x[b * rlb + k] = epilogue(epi, x[b * rlb + k], p[b * rlb + k], V[b * rlb + k], s);
-          if constexpr (sizeof(R) == 8) {
-            if (epi.so_map) {  // uniform: spinor filters only
-              const int u = epi.so_map[gi];
-              if (u >= 0) {  // vector v: spinor v / 2, up (v even) or down
-                const double *gq = epi.so_g + ((long)u * epi.so_nsp + (vec >> 1)) * 4 + 2 * (vec & 1);
-                x[b * rlb + k].re = fma(epi.so_alpha, gq[0], (double)x[b * rlb + k].re);
-                x[b * rlb + k].im = fma(epi.so_alpha, gq[1], (double)x[b * rlb + k].im);
-              }
-            }
-          }
           out.st(vec, gi, x[b * rlb + k]);
         }
     }
@@ -754,8 +668,7 @@ __global__ void __launch_bounds__(T) k_plane_bwd_fwd_w(cx<R> *tb, VecView<R> pin
 }
 
 // Pass C fused with the next pass A, with the plane held in registers and
-// transposed through a buffer of NX/NH columns: k_plane_bwd_w's and
-// k_plane_fwd_w's chunked forms back to back, same arithmetic as
+// transposed through a buffer of NX/NH columns, same arithmetic as
 // k_plane_bwd_fwd_w.  The buffer is 1/NH of a plane, so NH = 2 at complex64
 // 128^2 (67 KB) lets two workgroups share a CU and one's HBM phases run
 // under the other's FFTs; waves_per_eu holds the register budget to what two
@@ -929,7 +842,7 @@ k_plane_bwd_fwd_h(cx<R> *tb, VecView<R> pin, VecView<R> out, Epi<R> epi, long N,
 // ================================================================= dispatch
 template <typename R, int NX>
 constexpr size_t plane_lds() {
-  return sizeof(cx<R>) * ((size_t)NX * PlaneLds<R, NX, plane_chunks<R, NX>()>::LDc + NX);
+  return sizeof(cx<R>) * ((size_t)NX * PlaneLds<R, NX, 1>::LDc + NX);
 }
 
 template <typename R>

@@ -396,11 +396,12 @@ k_xrows_fwd(VecView<R> in, cx<R> *tb, int npair, int by, long N, const cx<R> *tw
   q.fwd(v, lds, tw, tb + vec * N, (unsigned)pi * (2 * AY * NX), gact);
 }
 
-// Sums of a workgroup's four partial sums per thread (T threads, any
-// multiple of 16) in fixed order: part[blk * 4 + q].
+// Sums of a workgroup's four partial sums per thread (T threads, 64 or more:
+// one whole wave adds them up) in fixed order: part[blk * 4 + q].
 template <int T>
 __device__ __forceinline__ void block_sum4_any(const double s[4], double *part, long blk,
                                                double *red) {
+  static_assert(T >= 64, "one whole wave adds the sums");
   lds_sync();
 #pragma unroll
   for (int q = 0; q < 4; q++) red[q * T + threadIdx.x] = s[q];
