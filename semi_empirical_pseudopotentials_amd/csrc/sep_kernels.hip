@@ -74,12 +74,14 @@ __global__ void __launch_bounds__(256) k_build_potential(
       z = xyz[3 * a + 2];
       ty = type[a];
       // beyond the last segment a pair adds nothing; the margin covers the
-      // rounding of the distance, the segment index below decides
+      // rounding of the distance, the segment index below decides.  An atom with
+      // a NaN coordinate is at no distance from any point: it is kept in every
+      // brick and makes all of V NaN
       const double rc = (double)(npot[ty] - 1) * dr[ty];
       rc2 = rc * rc * (1.0 + 1.0e-9);
       const double ex = fmax(fmax(x0 - x, x - x1), 0.0), ey = fmax(fmax(y0 - y, y - y1), 0.0),
                    ez = fmax(fmax(z0 - z, z - z1), 0.0);
-      keep = !(ex * ex + ey * ey + ez * ez > rc2);
+      keep = !(ex * ex + ey * ey + ez * ez > rc2) || x != x || y != y || z != z;
     }
     const unsigned long mask = __ballot(keep);
     __syncthreads();  // the previous atoms are consumed
