@@ -33,6 +33,8 @@
 // densities loaded ahead of the geometry).
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "sep_internal.h"
 
 namespace sep {
@@ -278,13 +280,26 @@ static int hf_pass(const GridDev &gd, double xmin, double ymin, double zmin, dou
   return hipGetLastError() == hipSuccess ? SEP_OK : SEP_ERR_HIP;
 }
 
-// Slices per atom: enough items for the persistent grid to balance (four per
-// workgroup), none below 1024 points of a box of `box` points.
-int hf_slices(long natom, double box) {
-  long n = (4L * HF_BLOCKS + natom - 1) / natom;
-  const long most = (long)(box / 1024.0) + 1;
-  if (n > most) n = most;
-  return (int)(n > 64 ? 64 : n);
+// Slices per atom of about `box` points, for passes of pb pairs: the least of
+// the persistent grid's work, halfway between its longest workgroup's share (x
+// rounded up) and the average (x).  A slice's reduction costs as much as some
+// 512 (pb + 1) points (3.5 us at one pair, 19 at eight), so that many slices
+// help a few atoms only: 100 atoms on 64^3 with 1 / 5 / 20 / 64 slices, whole
+// call: 8 pairs 334 / 306 / 361 / 543 us, one 253 / 228 / 233 / 272; 693 atoms
+// and 8 pairs with 1 / 2 / 4 / 64 448 / 471 / 521 / 2083; 10 atoms and 8 pairs
+// with 1 / 5 / 20 / 64 315 / 260 / 252 / 287.
+int hf_slices(long natom, double box, int pb) {
+  int best = 1;
+  double least = 0.0;
+  for (int n = 1; n <= 64; n++) {
+    const double x = (double)natom * n / HF_BLOCKS;
+    const double cost = (x + std::ceil(x)) * (box / n + 512.0 * (pb + 1));
+    if (n == 1 || cost < least) {
+      best = n;
+      least = cost;
+    }
+  }
+  return best;
 }
 
 // Pairs of one pass: the largest batch whose LDS histogram (pairs x maxnpot
@@ -303,9 +318,10 @@ int hf_adjoint_dev(const GridDev &gd, double xmin, double ymin, double zmin, dou
                    const double *pot, long stride, const double *dr, int ntype, const double *rho,
                    int np, int nsplit, int interp, double *work, double *htab, double *dR,
                    double *dscale, hipStream_t st) {
-  const int pb = hf_pairs_per_pass(maxnpot, np);
-  if (pb == 0) return SEP_ERR_ARG;
-  for (int p0 = 0; p0 < np; p0 += pb) {
+  if (hf_pairs_per_pass(maxnpot, np) == 0) return SEP_ERR_ARG;
+  // the last pass at the width of what is left
+  for (int p0 = 0, pb = 0; p0 < np; p0 += pb) {
+    pb = hf_pairs_per_pass(maxnpot, np - p0);
     int rc;
     switch (pb) {
       case 8:

@@ -4,6 +4,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <mutex>
+#include <numeric>
 
 #include <cmath>
 #include <cstdarg>
@@ -2003,22 +2004,26 @@ extern "C" int sep_hf_adjoint(sep_ctx *c, long npairs, const long *pairs, const 
   double rmax = 0.0;
   for (int t = 0; t < ntype; t++)
     if (npot[t] >= 2 && (double)(npot[t] - 1) * dr[t] > rmax) rmax = (double)(npot[t] - 1) * dr[t];
-  const double box = (2.0 * rmax / c->dx + 1.0) * (2.0 * rmax / c->dy + 1.0) * (2.0 * rmax / c->dz + 1.0);
-  const long nsplit = hf_slices(natom, box);
-  std::vector<int> order(natom);  // atoms by type, so that a table's histogram stays in LDS
-  for (long i = 0; i < natom; i++) order[i] = (int)i;
-  std::stable_sort(order.begin(), order.end(), [type](int x, int y) { return type[x] < type[y]; });
+  const double box = std::min(2.0 * rmax / c->dx + 1.0, (double)c->gd.nx) *
+                     std::min(2.0 * rmax / c->dy + 1.0, (double)c->gd.ny) *
+                     std::min(2.0 * rmax / c->dz + 1.0, (double)c->gd.nz);
   const int pb = hf_pairs_per_pass(maxnpot, np);
-  DevBuf xyz_d, type_d, order_d, npot_d, vr_d, pot_d, dr_d, scale_d, pairs_d, w_d, rho_d, work_d, htab_d,
+  const long nsplit = hf_slices(natom, box, pb);
+  // types, then the atoms by type, so that a table's histogram stays in LDS
+  std::vector<int> type_order(type, type + natom);
+  type_order.resize(2 * natom);
+  int *order = type_order.data() + natom;
+  std::iota(order, order + natom, 0);
+  std::stable_sort(order, order + natom, [type](int x, int y) { return type[x] < type[y]; });
+  DevBuf xyz_d, type_d, npot_d, vr_d, pot_d, dr_d, scale_d, pairs_d, w_d, rho_d, work_d, htab_d,
       dR_d, ds_d;
   RCHK(dev_upload(c, xyz_d, xyz, sizeof(double) * 3 * natom));
-  RCHK(dev_upload(c, type_d, type, sizeof(int) * natom));
+  RCHK(dev_upload(c, type_d, type_order.data(), sizeof(int) * 2 * natom));
   RCHK(dev_upload(c, npot_d, npot, sizeof(long) * ntype));
   RCHK(dev_upload(c, vr_d, vr, sizeof(double) * ntype * stride));
   RCHK(dev_upload(c, pot_d, pot, sizeof(double) * ntype * stride));
   RCHK(dev_upload(c, dr_d, dr, sizeof(double) * ntype));
   if (scale) RCHK(dev_upload(c, scale_d, scale, sizeof(double) * natom));
-  RCHK(dev_upload(c, order_d, order.data(), sizeof(int) * natom));
   RCHK(dev_upload(c, pairs_d, pairs, sizeof(long) * 2 * npairs));
   if (weights) RCHK(dev_upload(c, w_d, weights, sizeof(double) * npairs));
   RCHK(dev_alloc(c, rho_d, sizeof(double) * np * N));
@@ -2030,7 +2035,7 @@ extern "C" int sep_hf_adjoint(sep_ctx *c, long npairs, const long *pairs, const 
   RCHK(pair_density_dev(c->states, N, pairs_d.as<long>(), w_d.as<double>(), (int)npairs,
                         rho_d.as<double>(), c->st));
   int rc = hf_adjoint_dev(c->gd, c->xmin, c->ymin, c->zmin, c->dx, c->dy, c->dz, c->dv, (int)natom,
-                          xyz_d.as<double>(), type_d.as<int>(), order_d.as<int>(),
+                          xyz_d.as<double>(), type_d.as<int>(), type_d.as<int>() + natom,
                           scale_d.as<double>(), npot_d.as<long>(), maxnpot, vr_d.as<double>(), pot_d.as<double>(), stride,
                           dr_d.as<double>(), ntype, rho_d.as<double>(), (int)np, (int)nsplit,
                           c->interp, work_d.as<double>(), htab_d.as<double>(), dR_d.as<double>(),

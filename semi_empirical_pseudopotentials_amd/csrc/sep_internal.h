@@ -194,7 +194,7 @@ int dots_dev_f(const float *a, long lda, const float *b, long ldb, long m, long 
 int pair_density_dev(const double *states, long N, const long *pairs_d, const double *w_d, int np,
                      double *rho, hipStream_t st);
 int hf_pairs_per_pass(long maxnpot, long np);
-int hf_slices(long natom, double box);
+int hf_slices(long natom, double box, int pb);
 // order: the atoms sorted by type
 int hf_adjoint_dev(const GridDev &gd, double xmin, double ymin, double zmin, double dx, double dy,
                    double dz, double dv, int natom, const double *xyz, const int *type,
