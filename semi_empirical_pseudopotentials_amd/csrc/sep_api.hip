@@ -2530,7 +2530,7 @@ static int spinor_dots(sep_ctx *c, const double *x, const double *y, long m, dou
 static int normalize_spinors(sep_ctx *c, double *x, long m) {
   if (m <= 0) return SEP_OK;
   const long n4 = 4 * c->gd.N, nb = (n4 + 16383) / 16384;
-  RCHK(ensure_scr(c, (size_t)nb * m + 2 * (size_t)m));
+  RCHK(ensure_scr(c, (size_t)nb * m + 4 * (size_t)m));  // spinor_dots' size: it must not move out
   double *out = c->scr + nb * m;
   RCHK(spinor_dots(c, x, x, m, out));
   std::vector<double> nrm(m);
