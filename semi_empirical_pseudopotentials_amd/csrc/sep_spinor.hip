@@ -340,16 +340,24 @@ static void so_contrib_launch(const SoLists &so, const double *in, long cs, long
     // more points a lane as long as the workgroups fill the chip: 8 spinors
     // at 128 / 64 points a workgroup 192 / 215 us with 465 atoms (1395
     // workgroups at 128), 62 / 46 with 140 (420); 3 spinors at 64 / 32 points
-    // 18 / 16 us with 36 atoms (180 workgroups at 64)
+    // 18 / 16 us with 36 atoms (180 workgroups at 64).  One or two spinors are
+    // bound by the stream of K, which half the threads draw faster (whole H of
+    // one spinor, 341 points: 465 atoms at 96^3 258 us with four halves a
+    // workgroup, 209 with two, 222 at 32 points; 200 at 64^3 134, 105, 114; 30
+    // at 24^3 70, 71, 63)
     const auto groups = [&](long pb) { return so.natom * ((so.maxn + pb - 1) / pb); };
     if (nsp > 4 && groups(128) * ((nsp + 7) / 8) >= 1024)
       launch(k_so_contrib_k<4, 8>, 128, 8);
     else if (nsp > 4)
       launch(k_so_contrib_k<2, 8>, 64, 8);
-    else if (groups(64) >= 256)
+    else if (nsp > 2 && groups(64) >= 256)
       launch(k_so_contrib_k<2, 4>, 64, 4);
-    else
+    else if (nsp > 2)
       launch(k_so_contrib_k<1, 4>, 32, 4);
+    else if (groups(64) >= 1024)
+      launch(k_so_contrib_k<2, 2>, 64, 2);
+    else
+      launch(k_so_contrib_k<1, 2>, 32, 2);
   } else {
     hipLaunchKernelGGL(k_so_contrib, dim3((unsigned)so.natom, (unsigned)nsp), dim3(SO_T), 0, st,
                        so, in, cs, ss, contrib, nsp);
