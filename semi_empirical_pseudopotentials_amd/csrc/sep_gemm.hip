@@ -219,28 +219,43 @@ __global__ void __launch_bounds__(512) k_sum_chunks(const double *work, long nch
 }
 
 // Shape of one Gram launch.  Block tile GT x bw; chunk count a multiple of 8
-// (one group per XCD) giving >= ~2048 blocks.  A chunk has at least 4096
+// (one group per XCD) of at most ~2048 blocks in all.  A chunk has at least 4096
 // contraction indices, or fewer for few states, whose single tile would leave
 // most CUs idle: so many that a chunk reads 16 times the bytes of its partial
 // sums, and 64 MB of partial sums in all.  64 states of 48^3 in FP64 with 32
 // workgroups 433 us, with 216 70 us; the whole call in FP32 at 64 states of
-// 128^3 776 -> 383 us (at 256 states the chunks are as before).
+// 128^3 776 -> 383 us.  Several tiles take that, the 4096 indices or as many
+// chunks as fill the CUs once, whichever leaves the least of the last round of
+// workgroups idle (an XCD holds 32 at once in FP64, 64 in FP32), the fewer
+// where they tie: 200 states of 64^3, four tiles, with 64 / 128 / 168 / 256
+// chunks FP64 662 / 664 / 734 / 685 us, FP32 401 / 371 / 411 / 383; 384 states of
+// 48^3 in FP64 with 32 / 40 chunks 970 / 801.
 struct GramShape {
   int tj, ntiles, nch;
   long kc;
 };
-static GramShape gram_shape(long m, long mb, long K, bool sym, int bw) {
+static GramShape gram_shape(long m, long mb, long K, bool sym, int bw, bool fp64) {
   GramShape g;
   const int ti = (int)((m + GT - 1) / GT);
   if (sym) bw = GT;  // square tiles on the diagonal
   g.tj = (int)((mb + bw - 1) / bw);
   g.ntiles = sym ? ti * (ti + 1) / 2 : ti * g.tj;
-  long want = (2048 + g.ntiles - 1) / g.ntiles;
+  const long most = (2048 + g.ntiles - 1) / g.ntiles;
   const long kmin = std::max(512L, 16 * m * mb / (m + mb));
-  long maxch = std::max((K + 4095) / 4096, std::min((K + kmin - 1) / kmin, (8L << 20) / (m * mb)));
-  if (want > maxch) want = maxch;
-  if (want < 1) want = 1;
-  want = (want + 7) / 8 * 8;
+  const long fine = std::min((K + kmin - 1) / kmin, (8L << 20) / (m * mb));
+  auto chunks = [&](long n) { return (std::max(1L, std::min(n, most)) + 7) / 8 * 8; };
+  const long coarse = (K + 4095) / 4096;
+  long want = chunks(std::max(coarse, fine));
+  if (g.ntiles > 1) {
+    const long slots = fp64 ? 32 : 64;
+    // rounds of workgroups on an XCD, per chunk
+    auto rounds = [&](long n) {
+      return (double)((n / 8 * g.ntiles + slots - 1) / slots) / (double)n;
+    };
+    for (long n : {chunks(std::max(coarse, std::min(fine, 8 * slots / g.ntiles / 8 * 8))),
+                   chunks(coarse)})
+      if (rounds(n) < rounds(want) || (rounds(n) == rounds(want) && n < want)) want = n;
+  }
   g.kc = (K + want - 1) / want;
   g.kc = (g.kc + GKB - 1) / GKB * GKB;
   g.nch = (int)((K + g.kc - 1) / g.kc);
@@ -269,10 +284,8 @@ struct GramCfg<float> {
 long gram_work_len(long m, long mb, long K) {
   long n = 0;
   for (int bw : {32, 64, 128})
-    for (bool sym : {false, true}) {
-      const GramShape g = gram_shape(m, mb, K, sym, bw);
-      if (g.nch > n) n = g.nch;
-    }
+    for (bool sym : {false, true})
+      for (bool fp64 : {false, true}) n = std::max<long>(n, gram_shape(m, mb, K, sym, bw, fp64).nch);
   return n * m * mb;
 }
 
@@ -280,7 +293,7 @@ template <typename R, int TJ, int ST>
 int gram_launch(const R *A, long lda, long m, const R *B, long ldb, long mb, long K, bool sym,
                 double *C_d, double *work, long work_len, hipStream_t st) {
   if (sym && (m != mb || TJ != 4)) return SEP_ERR_ARG;
-  const GramShape g = gram_shape(m, mb, K, sym, 32 * TJ);
+  const GramShape g = gram_shape(m, mb, K, sym, 32 * TJ, sizeof(R) == 8);
   if ((long)g.nch * m * mb > work_len) return SEP_ERR_NOMEM;
   const int ngrp = (g.nch + 7) / 8;
   const unsigned nblk = (unsigned)(8 * ngrp * g.ntiles);
