@@ -21,6 +21,23 @@
 #include "../../include/sep_deck.h"
 #include "sep_host.h"
 
+/* ======================================================== OpenMP teams */
+/* LLVM's runtime lets a team's threads spin for a while after each region (200
+ * ms): what the loops of many short regions here want between them, and what the
+ * caller's own threads pay for afterwards (the first conversion of a filtered
+ * block to float on 16 threads 0.1 -> 6 ms).  One more region with no such time
+ * sends the team to sleep; other runtimes do not have the call. */
+extern void kmp_set_blocktime(int) __attribute__((weak));
+extern int kmp_get_blocktime(void) __attribute__((weak));
+static void team_rest(void) {
+  if (!kmp_set_blocktime || !kmp_get_blocktime) return;
+  const int ms = kmp_get_blocktime();
+  kmp_set_blocktime(0);
+#pragma omp parallel
+  { __asm__ volatile("" ::: "memory"); }
+  kmp_set_blocktime(ms);
+}
+
 /* ======================================================= copy threads */
 /* A copy is cut into pieces that whoever runs takes in turn, the caller
  * included: threads that the machine gives no CPU yet (the caller's own busy
@@ -314,6 +331,7 @@ double sep_leja_points(long nc, double *zn) {
   for (long j = 0; j < nc; j++) prod *= pre[j] * pre[j];
   double fk = pow(sqrt(prod), 1.0 / (double)nc);
   memcpy(zn, pre, sizeof(double) * nc);
+  team_rest();
   free(cre);
   free(score);
   free(pre);
@@ -345,6 +363,7 @@ int sep_newton_coeffs(long nc, long ms, const double *zn, const double *el, doub
       a[j] = (fj - a[0] - acc) / w;
     }
   }
+  team_rest();
   return SEP_OK;
 }
 
@@ -414,6 +433,7 @@ int sep_la_chol_dd(long n, const double *hi, const double *lo, double shift, dou
       R[j * n + c] = dd_div(s, rjj);
     }
   }
+  if (n > 64) team_rest();
   for (long i = 0; i < n; i++)
     for (long j = 0; j < n; j++) Rout[i * n + j] = (j >= i && !status) ? R[i * n + j].hi : 0.0;
   free(R);
