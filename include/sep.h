@@ -166,7 +166,7 @@ int sep_filter_dev(sep_ctx *ctx, const void *psi0_dev, long ns, const double *an
 /* ------------------------------------------------- dense device contractions */
 /* On device buffers of the context's grid (N = nx ny nz points per state,
  * state-major; FP64 when precision = SEP_PREC_FP64, FP32 otherwise), on the
- * matrix cores (FP64: rocBLAS dgemm; FP32: this library's MFMA kernels):
+ * matrix cores (this library's MFMA kernels in both precisions):
  *   sep_gram_dev    C[i][j] = sum_g A[i][g] B[j][g]   (C: host, m x mb, FP64)
  *   sep_rotate_dev  Out[j][g] = sum_i M[i][j] A[i][g] (M: host, m x mo row-major)
  * They are the projected-H / overlap contractions and the Ritz rotation of

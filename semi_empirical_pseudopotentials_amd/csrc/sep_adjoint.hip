@@ -20,7 +20,8 @@
 // is continuous.
 //
 // Work split: an item is a slice of one atom's bounding box of grid points
-// within the table range; a persistent grid of two workgroups per CU takes
+// within the table range (as many slices as make the runs of items even, a few
+// long ones for few atoms: hf_slices); a persistent grid of two workgroups per CU takes
 // contiguous runs of items, atoms sorted by type.  An item's partial sums go
 // to a work array, summed in slice order by a second kernel.  The table
 // histogram accumulates in LDS over all of a workgroup's items of one type and
@@ -28,9 +29,9 @@
 // only).  Bound by the FP64 divisions and square root of a point, its LDS
 // atomics and the few waves that the histogram's LDS leaves on a CU (77 KB
 // for 8 pairs of 1201 rows).  693 atoms on 96^3, linear tables: one density
-// 186 us (539 with a workgroup per slice), 3 pairs 251 (730), 8 pairs 430
+// 178 us (539 with a workgroup per slice), 3 pairs 232 (730), 8 pairs 381
 // (1179; 748 before the row weights were specialised by interpolation and the
-// densities loaded ahead of the geometry).
+// densities loaded ahead of the geometry), 8 pairs of cubic tables 693.
 #include <hip/hip_runtime.h>
 
 #include <cmath>

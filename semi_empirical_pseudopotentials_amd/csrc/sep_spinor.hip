@@ -175,8 +175,11 @@ __global__ void __launch_bounds__(SO_T) k_so_kmat(SoLists so) {
 // the LDS reads, 12 + PT words a lane for 12 PT multiply-adds.  465 atoms of 244-277
 // points at 96^3 (8 spinors: 5.5 GFLOP FP64, 85 us at the VALU's rate), in us
 // at 8 / 4 / 2 / 1 spinors: one point a lane and K from L2 273 / 161 / 115 /
-// 105, now 192 / 129 / 102 / 96.  K on the matrix cores would not help: their
-// FP64 rate is below the VALU's here (sep_gemm.hip).  Skipping the 32-point
+// 105, now 192 / 129 / 93 / 85 (workgroups of two spinors for the last two: with
+// half-empty ones of four 102 / 96).  K on the matrix cores is not tried:
+// v_mfma_f64_16x16x4 issues 36-48 TFLOP/s from registers alone, FP64 FMAs 65,
+// and this product reaches 29, so fewer LDS words a product could still pay
+// there.  Skipping the 32-point
 // rows past the list by a branch stops the LDS reads from running ahead (293).
 // Workgroup b runs on XCD b % 8; an atom's workgroups share that XCD.  Each
 // point's sums run over q in the order of k_so_contrib: bit for bit the same.
